@@ -170,6 +170,22 @@ constexpr bool stores(bool fin, int r, int lane, int l, int lines_here, int lone
 constexpr uint32_t kBufWord3 = 0x00020000;  // raw dword buffer, gfx9 family
 constexpr uint32_t kOutOfRange = 0xF0000000u;
 
+// IL: coefficients in interleaved order, each at the position of the sample it
+// replaces (lifting in place): detail k of level l at (2k + 1) 2^(LEV-1-l), the
+// coarse block at multiples of 2^(LEV-2).  A line is then transformed in place:
+// the forward stores details only at positions it has read, the inverse
+// samples only at positions whose coefficient it has read.
+template <bool IL, int LEV, int EXT>
+constexpr int coef_pos(int i) {
+    if (!IL) return i;
+    if (i < 4 + EXT) return i << (LEV - 2);
+    int l = 2;
+    while (i - EXT >= (2 << l)) ++l;
+    return (2 * (i - EXT - (1 << l)) + 1) << (LEV - 1 - l);
+}
+
+// FWD: loads are samples and stores coefficients; the inverse the other way.
+template <bool IL, int LEV, int EXT, bool FWD>
 struct StridedIO {
     static constexpr int kLook = WHHD_LOOK_S;  // samples loaded ahead of use
     static constexpr bool kTwoPhase = false;   // loads land in the line registers directly
@@ -181,7 +197,8 @@ struct StridedIO {
     int step_bytes;
     int n;
     WHHD_DEV float load(int i) const {
-        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff_ld, i * step_bytes, 0));
+        const int at = FWD ? i : coef_pos<IL, LEV, EXT>(i);
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff_ld, at * step_bytes, 0));
     }
     // The stores' scalar offsets come from step_st, an opaque copy of
     // step_bytes in the forward: otherwise the compiler keeps every load's
@@ -190,8 +207,9 @@ struct StridedIO {
     // each) instead of multiplying again.
     int step_st;
     WHHD_DEV void store(int i, float v) const {
+        const int at = FWD ? coef_pos<IL, LEV, EXT>(i) : i;
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rd, voff_st,
-                                              i * step_st, 0);
+                                              at * step_st, 0);
     }
     // samples [START, START+CNT) of the line; each store is already one row
     template <int START, int CNT>
@@ -532,7 +550,8 @@ WHHD_DEV void fwd_levels_below(const IO& io, float* in) {
             float acc = 0.f;
             static_for<0, M>([&](auto ci) {
                 constexpr int c = decltype(ci)::value;
-                acc += in[c] * float(W::l10[r * M + c]);
+                constexpr float m = float(W::l10[r * M + c]);  // an immediate, not a load
+                acc += in[c] * m;
             });
             run[r] = acc;
         });
@@ -693,7 +712,8 @@ WHHD_DEV void inverse_line_lp(const IO& io) {
         float acc = 0.f;
         static_for<0, M>([&](auto ci) {
             constexpr int cc = decltype(ci)::value;
-            acc += x[cc] * float(W::il10[r * M + cc]);
+            constexpr float m = float(W::il10[r * M + cc]);
+            acc += x[cc] * m;
         });
         a[r] = acc;
     });
@@ -710,84 +730,126 @@ WHHD_DEV void inverse_line_lp(const IO& io) {
 // inner * inner_stride + outer * outer_stride and its samples are `step` apart.
 // Problems of a batch are arrays of equal extents `batch_stride` elements
 // apart; grid row blockIdx.y transforms problem blockIdx.y.
+// (Everything inside one array fits 32-bit byte offsets.)
 struct LpGeom {
-    int64_t total_lines;
-    int64_t total_elems;  // elements in one problem's array (buffer range)
-    int lines_inner;
-    int64_t inner_stride;
-    int64_t outer_stride;
-    int64_t step;
+    uint32_t total_lines;
+    uint32_t total_elems;  // elements in one problem's array (buffer range)
+    uint32_t lines_inner;
+    uint32_t inner_stride;
+    uint32_t outer_stride;
+    uint32_t step;
     int64_t batch_stride;
 };
 
-template <class W, int LEV, int EXT, bool FWD, bool CONTIG>
-// Two wavefronts per SIMD: a pass over 256^3 has about one wavefront of lines
-// per SIMD, so the register budget goes to loads in flight, not occupancy.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-lp_kernel(float* __restrict__ dst, const float* __restrict__ src, LpGeom g) {
-    src += (int64_t)blockIdx.y * g.batch_stride;
-    dst += (int64_t)blockIdx.y * g.batch_stride;
-    // Workgroups go to the 8 XCDs round-robin (blockIdx.x % 8), each XCD with
-    // its own L2; give every XCD a contiguous run of tiles, so that the cache
-    // lines two neighbouring tiles share (rows of 2^L + 1 floats start
-    // unaligned) are fetched and written through one L2.
-    const unsigned nwg = gridDim.x, bxr = blockIdx.x % 8u, bxq = blockIdx.x / 8u;
-    const unsigned tile = bxr * (nwg / 8u) + (bxr < nwg % 8u ? bxr : nwg % 8u) + bxq;
+// A launch transforms up to three arrays along one axis (the components of a
+// velocity or potential): `kind` 0 with the curl wavelet WC on 2^LEV samples,
+// 1 with the divergence wavelet WD on 2^LEV + 1.
+constexpr int kMaxJobs = 3;
+struct LpJob {
+    float* dst;
+    const float* src;
+    LpGeom g;
+    unsigned tiles;  // workgroups
+    int kind;
+};
+struct LpJobs {
+    LpJob j[kMaxJobs];
+    int n;
+};
+
+enum Layout { kContig = 0, kStrided = 1, kInterleaved = 2 };
+
+template <class W, int LEV, int EXT, bool FWD, int LAY>
+WHHD_DEV void lp_tile(const LpJob& jb, unsigned tile) {
+    const LpGeom& g = jb.g;
+    const float* src = jb.src + (int64_t)blockIdx.y * g.batch_stride;
+    float* dst = jb.dst + (int64_t)blockIdx.y * g.batch_stride;
     const int lane_ = threadIdx.x & 63;
     const int64_t wave_first = ((int64_t)tile * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64;
     const int64_t li = wave_first + lane_;
     const bool valid = li < g.total_lines;  // lanes past the last line load line 0, never store
-    const int64_t l = valid ? li : 0;
-    const int64_t outer = l / g.lines_inner;
-    const int64_t inner = l - outer * g.lines_inner;
+    const uint32_t l = valid ? (uint32_t)li : 0u;
     constexpr int n = (1 << LEV) + EXT;
-    const uint32_t bytes = (uint32_t)(g.total_elems * 4);
+    const uint32_t bytes = g.total_elems * 4;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, bytes, kBufWord3);
     const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)dst, 0, bytes, kBufWord3);
-    if constexpr (CONTIG) {
+    if constexpr (LAY == kContig) {
         // contiguous lines are numbered in memory order: line li starts at li * n
         // one staging area of kStageRun x kStageRow per wavefront (dynamic
         // LDS), three for the inverse's aligned stores
         extern __shared__ __attribute__((aligned(16))) float lp_stage[];
         constexpr int kWaveStage = (!FWD && tail::applies<n>() ? tail::kAreas : 1) * kStageRun * kStageRow;
-        const int64_t here = g.total_lines - wave_first;
-        const uint32_t voff = (uint32_t)(l * n * 4);
-        ContigIO io{src + l * n, rs, rd, valid ? voff : kOutOfRange,
+        const int64_t here = (int64_t)g.total_lines - wave_first;
+        const uint32_t voff = l * n * 4;
+        ContigIO io{src + (int64_t)l * n, rs, rd, valid ? voff : kOutOfRange,
                     (uint32_t)(wave_first * n * 4), (int)(here < 64 ? here : 64), n,
                     lp_stage + (threadIdx.x >> 6) * kWaveStage, lane_};
         if (FWD) forward_line_lp<W, LEV, EXT>(io);
         else inverse_line_lp<W, LEV, EXT>(io);
     } else {
-        const uint32_t voff = (uint32_t)((inner * g.inner_stride + outer * g.outer_stride) * 4);
-        int step_st = (int)(g.step * 4);
-        if constexpr (FWD) asm volatile("s_mov_b32 %0, %0" : "+s"(step_st));
-        StridedIO io{rs, rd, voff, valid ? voff : kOutOfRange, (int)(g.step * 4), n, step_st};
+        const uint32_t outer = l / g.lines_inner;
+        const uint32_t inner = l - outer * g.lines_inner;
+        const uint32_t voff = (inner * g.inner_stride + outer * g.outer_stride) * 4;
+        // opaque to the compiler here: it would otherwise form the offsets
+        // i * step that the two wavelets' bodies share ahead of the branch
+        // between them and spill them (170-360 SGPRs, 256^3 solve 659 -> 695 us)
+        int step = (int)(g.step * 4);
+        asm volatile("s_mov_b32 %0, %0" : "+s"(step));
+        int step_st = step;
+        asm volatile("s_mov_b32 %0, %0" : "+s"(step_st));
+        StridedIO<LAY == kInterleaved, LEV, EXT, FWD> io{rs, rd, voff, valid ? voff : kOutOfRange, step, n, step_st};
         if (FWD) forward_line_lp<W, LEV, EXT>(io);
         else inverse_line_lp<W, LEV, EXT>(io);
     }
 }
 
-// Launch the line-parallel kernel for `levels` (5..8) over `nb` problems with
+template <class WC, class WD, int LEV, bool FWD, int LAY>
+// Two wavefronts per SIMD: a pass over 256^3 has about one wavefront of lines
+// per SIMD, so the register budget goes to loads in flight, not occupancy.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+lp_kernel(LpJobs a) {
+    const LpJob& jb = a.j[blockIdx.z];
+    // Workgroups go to the 8 XCDs round-robin (blockIdx.x % 8), each XCD with
+    // its own L2; give every XCD a contiguous run of tiles, so that the cache
+    // lines two neighbouring tiles share (rows of 2^L + 1 floats start
+    // unaligned) are fetched and written through one L2.
+    const unsigned nwg = jb.tiles, bxr = blockIdx.x % 8u, bxq = blockIdx.x / 8u;
+    if (blockIdx.x >= nwg) return;  // a grid row is as long as the largest job's
+    const unsigned tile = bxr * (nwg / 8u) + (bxr < nwg % 8u ? bxr : nwg % 8u) + bxq;
+    if (jb.kind == 0) lp_tile<WC, LEV, 0, FWD, LAY>(jb, tile);
+    else lp_tile<WD, LEV, 1, FWD, LAY>(jb, tile);
+}
+
+// Launch the line-parallel kernel for `levels` (3..8) over `nb` problems with
 // `waves` (1, 2 or 4) wavefronts per workgroup; false if none exists.
-template <class W, int EXT, bool FWD, bool CONTIG>
-bool lp_launch_one(int levels, float* dst, const float* src, const LpGeom& g, int waves, int nb,
-                   hipStream_t s) {
+template <class WC, class WD, bool FWD, int LAY>
+bool lp_launch_one(int levels, LpJobs& a, int waves, int nb, hipStream_t s) {
     if (waves != 1 && waves != 2 && waves != 4) return false;
-    if (nb < 1 || nb > 65535) return false;
+    if (nb < 1 || nb > 65535 || a.n < 1 || a.n > kMaxJobs) return false;
     const dim3 block(64 * waves);
     const int64_t lines_per_block = 64 * waves;
-    const dim3 grid((unsigned)((g.total_lines + lines_per_block - 1) / lines_per_block), (unsigned)nb);
-    // the inverse of lines of 2^levels + 1 samples stores through three runs
-    const int n = (1 << levels) + EXT;
-    const int rows = !FWD && n % 32 == 1 && n >= 33 ? tail::kAreas * kStageRun : kStageRun;
-    const size_t lds = CONTIG ? (size_t)waves * rows * kStageRow * sizeof(float) : 0;
+    int64_t tiles = 0;  // of the largest job
+    int rows = kStageRun;
+    for (int k = 0; k < a.n; ++k) {
+        const int64_t t = ((int64_t)a.j[k].g.total_lines + lines_per_block - 1) / lines_per_block;
+        a.j[k].tiles = (unsigned)t;
+        tiles = t > tiles ? t : tiles;
+        // the inverse of lines of 2^levels + 1 samples stores through three runs
+        const int n = (1 << levels) + a.j[k].kind;
+        if (!FWD && n % 32 == 1 && n >= 33) rows = tail::kAreas * kStageRun;
+    }
+    if (tiles < 1 || tiles > 0x7fffffff - 8) return false;
+    // rows of a multiple of 8 workgroups keep blockIdx.x % 8 the XCD in every row
+    if (a.n > 1) tiles = (tiles + 7) / 8 * 8;
+    const dim3 grid((unsigned)tiles, (unsigned)nb, (unsigned)a.n);
+    const size_t lds = LAY == kContig ? (size_t)waves * rows * kStageRow * sizeof(float) : 0;
+#define WHHD_LP(LEV) \
+    case LEV: hipLaunchKernelGGL((lp_kernel<WC, WD, LEV, FWD, LAY>), grid, block, lds, s, a); return true;
     switch (levels) {
-    case 5: hipLaunchKernelGGL((lp_kernel<W, 5, EXT, FWD, CONTIG>), grid, block, lds, s, dst, src, g); return true;
-    case 6: hipLaunchKernelGGL((lp_kernel<W, 6, EXT, FWD, CONTIG>), grid, block, lds, s, dst, src, g); return true;
-    case 7: hipLaunchKernelGGL((lp_kernel<W, 7, EXT, FWD, CONTIG>), grid, block, lds, s, dst, src, g); return true;
-    case 8: hipLaunchKernelGGL((lp_kernel<W, 8, EXT, FWD, CONTIG>), grid, block, lds, s, dst, src, g); return true;
+        WHHD_LP(3) WHHD_LP(4) WHHD_LP(5) WHHD_LP(6) WHHD_LP(7) WHHD_LP(8)
     default: return false;
     }
+#undef WHHD_LP
 }
 
 #endif  // WHHD_HOST_EMULATION
@@ -795,14 +857,13 @@ bool lp_launch_one(int levels, float* dst, const float* src, const LpGeom& g, in
 }  // namespace lp
 
 #ifndef WHHD_HOST_EMULATION
-template <class W, int EXT>
-bool lp_launch(int levels, bool fwd, bool contig, float* dst, const float* src,
-               const lp::LpGeom& g, int waves, int nb, hipStream_t s) {
-    if (contig)
-        return fwd ? lp::lp_launch_one<W, EXT, true, true>(levels, dst, src, g, waves, nb, s)
-                   : lp::lp_launch_one<W, EXT, false, true>(levels, dst, src, g, waves, nb, s);
-    return fwd ? lp::lp_launch_one<W, EXT, true, false>(levels, dst, src, g, waves, nb, s)
-               : lp::lp_launch_one<W, EXT, false, false>(levels, dst, src, g, waves, nb, s);
+template <class WC, class WD, bool FWD>
+bool lp_launch(int levels, int layout, lp::LpJobs& a, int waves, int nb, hipStream_t s) {
+    switch (layout) {
+    case lp::kContig: return lp::lp_launch_one<WC, WD, FWD, lp::kContig>(levels, a, waves, nb, s);
+    case lp::kStrided: return lp::lp_launch_one<WC, WD, FWD, lp::kStrided>(levels, a, waves, nb, s);
+    default: return lp::lp_launch_one<WC, WD, FWD, lp::kInterleaved>(levels, a, waves, nb, s);
+    }
 }
 
 #endif  // WHHD_HOST_EMULATION

@@ -277,8 +277,8 @@ int transform_lines(T* dst, const T* src, int nx, int ny, int nz, int levels, ch
     if (st != WHHD_OK) return st;
     if constexpr (sizeof(T) == sizeof(float)) {
         if ((!cfg || cfg->allow_line_parallel) && g_line_kernel_mode.load() == 0) {
-            const int r = lp_transform((float*)dst, (const float*)src, nx, ny, nz, levels, axis, bc,
-                                       wt, fwd, stream, b);
+            const LineJob job{(float*)dst, (const float*)src, nx, ny, nz, bc, wt, b.stride};
+            const int r = lp_transform(&job, 1, levels, axis, fwd, false, stream, b.waves, b.nb);
             if (r != -1) return r;
         }
     }

@@ -74,6 +74,7 @@ struct Proj3Args {
     AxisCoef cx, cy, cz;
     int nx, ny, nz;
     int zblocks;  // grid z rows per problem
+    int qx4, qz4;  // interleaved: nx / 4, nz / 4
     int64_t bv[3], bq[3];
     int nq;                       // divergence bc 'n' boundary cells
     float lix, liy, liz;          // 1 / domain length per axis
@@ -84,7 +85,13 @@ struct Proj3Args {
 // within the workgroup; offsets in index type I (32-bit whenever every array
 // fits).  Tile row tz covers z block (tz % zblocks) of problem
 // (tz / zblocks).
-template <class I, int ZB>
+//
+// IL: along x and z the coefficients lie interleaved (line_parallel.h), curl-type
+// index c at position coef_pos(c) and divergence-type c + 1 at the same position
+// for a detail, a quarter of the extent further on for the coarse block; x and z
+// below are positions, the coefficient rows are in that order, and index 0 is
+// position 0 of either type.
+template <class I, int ZB, bool IL>
 __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
     // workgroups go to the 8 XCDs round-robin in launch order; each XCD takes a
     // contiguous run of tiles, so rows that share a cache line share an L2
@@ -109,12 +116,15 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
     const I sqx_x = NY + 1, sqx_z = NX * (NY + 1);
     const I sqy_x = NY, sqy_z = (NX + 1) * NY;
     const I sqz_x = NY + 1, sqz_z = (NX + 1) * (NY + 1);
-    I ixv = y + (x + 1) * NY + z0 * sxv_z;
+    // where divergence-type coefficient c + 1 of curl-type c lies
+    auto next = [](int c, int q4) -> I { return IL ? c + ((c & (q4 - 1)) == 0 ? q4 : 0) : c + 1; };
+    const I xd = next(x, p.qx4);
+    I ixv = y + xd * NY + z0 * sxv_z;
     I iyv = (y + 1) + x * (NY + 1) + z0 * syv_z;
-    I izv = y + x * NY + (z0 + 1) * szv_z;
-    I iqx = (y + 1) + x * sqx_x + (z0 + 1) * sqx_z;
-    I iqy = y + (x + 1) * sqy_x + (z0 + 1) * sqy_z;
-    I iqz = (y + 1) + (x + 1) * sqz_x + z0 * sqz_z;
+    const I jzv = y + x * NY;
+    const I jqx = (y + 1) + x * sqx_x;
+    const I jqy = y + xd * sqy_x;
+    I iqz = (y + 1) + xd * sqz_x + z0 * sqz_z;
     const float sx = p.cx.s[x], sy = p.cy.s[y];
     const float sxx_syy = sx * sx + sy * sy;
     const int zend = min(z0 + ZB, p.nz);
@@ -130,11 +140,11 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
 #if WHHD_PROJ_NT
         pvx[k] = __builtin_nontemporal_load(p.xv + ixv + kk * sxv_z);
         pvy[k] = __builtin_nontemporal_load(p.yv + iyv + kk * syv_z);
-        pvz[k] = __builtin_nontemporal_load(p.zv + izv + kk * szv_z);
+        pvz[k] = __builtin_nontemporal_load(p.zv + jzv + next(z0 + kk, p.qz4) * szv_z);
 #else
         pvx[k] = p.xv[ixv + kk * sxv_z];
         pvy[k] = p.yv[iyv + kk * syv_z];
-        pvz[k] = p.zv[izv + kk * szv_z];
+        pvz[k] = p.zv[jzv + next(z0 + kk, p.qz4) * szv_z];
 #endif
         psz[k] = p.cz.s[z0 + kk];
     }
@@ -142,6 +152,8 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
     for (int k = 0; k < ZB; ++k) {
         const int z = z0 + k;
         if (z >= zend) break;
+        const I zd = next(z, p.qz4);
+        const I izv = jzv + zd * szv_z, iqx = jqx + zd * sqx_z, iqy = jqy + zd * sqy_z;
         const float sz = psz[k];
         const float vx = pvx[k], vy = pvy[k], vz = pvz[k];
         float lx = 0.f, ly = 0.f, lz = 0.f;
@@ -151,6 +163,9 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
             lx = (sz * vy - sy * vz) * inv;
             ly = (sx * vz - sz * vx) * inv;
         } else {
+            // from index c + 1 (c = 0) back to index 0 along the divergence-type axes
+            const I ozv = zd * szv_z, oqx_z = zd * sqx_z, oqy_z = zd * sqy_z;
+            const I oxv = xd * NY, oqy_x = xd * sqy_x, oqz_x = xd * sqz_x;
             const float ip0x = p.cx.b0[x], ip1x = p.cx.b1[x];
             const float ip0y = p.cy.b0[y], ip1y = p.cy.b1[y];
             const float ip0z = p.cz.b0[z], ip1z = p.cz.b1[z];
@@ -158,13 +173,13 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
             if (p.nq) {
                 // index-0 samples of the in-plane components (read only where used)
                 if (x > 0 && y > 0 && z == 0) {
-                    const float z0 = p.zv[izv - szv_z];
+                    const float z0 = p.zv[izv - ozv];
                     const float sxBxBy = sx * ip0x * ip1y * ip0z;
                     const float syBxBy = sy * ip1x * ip0y * ip0z;
                     const float mz = 1.f / (sx * sxBxBy + sy * syBxBy + eps);
                     const float a0 = z0 / sx, a1 = vz / sx;
-                    p.qx[iqx - sqx_z] = 0.f;
-                    p.qy[iqy - sqy_z] = a0;
+                    p.qx[iqx - oqx_z] = 0.f;
+                    p.qy[iqy - oqy_z] = a0;
                     ly = a1;
                     const float vx2 = vx + (a1 - a0) * p.liz;
                     lz = (vx2 * syBxBy - vy * sxBxBy) * mz;
@@ -180,56 +195,56 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
                     ly = (vz2 * sxBxBz - vx * szBxBz) * my;
                     p.qz[iqz - 1] = 0.f;
                 } else if (y > 0 && z > 0 && x == 0) {
-                    const float x0 = p.xv[ixv - NY];
+                    const float x0 = p.xv[ixv - oxv];
                     const float syByBz = sy * ip0x * ip0y * ip1z;
                     const float szByBz = sz * ip0x * ip1y * ip0z;
                     const float mx = 1.f / (sy * syByBz + sz * szByBz + eps);
                     const float a0 = x0 / sy, a1 = vx / sy;
-                    p.qz[iqz - sqz_x] = a0;
+                    p.qz[iqz - oqz_x] = a0;
                     lz = a1;
                     const float vy2 = vy + (a1 - a0) * p.lix;
                     lx = (vy2 * szByBz - vz * syByBz) * mx;
-                    p.qy[iqy - sqy_x] = 0.f;
+                    p.qy[iqy - oqy_x] = 0.f;
                 } else if (x > 0 && y == 0 && z == 0) {
-                    const float y0 = p.yv[iyv - 1], z0 = p.zv[izv - szv_z];
-                    p.qy[iqy - sqy_z] = z0 / sx;
+                    const float y0 = p.yv[iyv - 1], z0 = p.zv[izv - ozv];
+                    p.qy[iqy - oqy_z] = z0 / sx;
                     ly = vz / sx;
                     p.qz[iqz - 1] = -y0 / sx;
                     lz = -vy / sx;
                     p.qx[iqx - 1] = 0.f;
-                    p.qx[iqx - sqx_z - 1] = 0.f;
-                    p.qx[iqx - sqx_z] = 0.f;
+                    p.qx[iqx - oqx_z - 1] = 0.f;
+                    p.qx[iqx - oqx_z] = 0.f;
                 } else if (y > 0 && x == 0 && z == 0) {
-                    const float z0 = p.zv[izv - szv_z], x0 = p.xv[ixv - NY];
-                    p.qx[iqx - sqx_z] = -z0 / sy;
+                    const float z0 = p.zv[izv - ozv], x0 = p.xv[ixv - oxv];
+                    p.qx[iqx - oqx_z] = -z0 / sy;
                     lx = -vz / sy;
-                    p.qz[iqz - sqz_x] = x0 / sy;
+                    p.qz[iqz - oqz_x] = x0 / sy;
                     lz = vx / sy;
-                    p.qy[iqy - sqy_x - sqy_z] = 0.f;
-                    p.qy[iqy - sqy_z] = 0.f;
-                    p.qy[iqy - sqy_x] = 0.f;
+                    p.qy[iqy - oqy_x - oqy_z] = 0.f;
+                    p.qy[iqy - oqy_z] = 0.f;
+                    p.qy[iqy - oqy_x] = 0.f;
                 } else if (z > 0 && x == 0 && y == 0) {
-                    const float y0 = p.yv[iyv - 1], x0 = p.xv[ixv - NY];
+                    const float y0 = p.yv[iyv - 1], x0 = p.xv[ixv - oxv];
                     p.qx[iqx - 1] = y0 / sz;
                     lx = vy / sz;
-                    p.qy[iqy - sqy_x] = -x0 / sz;
+                    p.qy[iqy - oqy_x] = -x0 / sz;
                     ly = -vx / sz;
-                    p.qz[iqz - sqz_x - 1] = 0.f;
-                    p.qz[iqz - sqz_x] = 0.f;
+                    p.qz[iqz - oqz_x - 1] = 0.f;
+                    p.qz[iqz - oqz_x] = 0.f;
                     p.qz[iqz - 1] = 0.f;
                 } else {
-                    const float y0 = p.yv[iyv - 1], x0 = p.xv[ixv - NY], z0 = p.zv[izv - szv_z];
-                    p.qz[iqz - 1 - sqz_x] = 0.f;
+                    const float y0 = p.yv[iyv - 1], x0 = p.xv[ixv - oxv], z0 = p.zv[izv - ozv];
+                    p.qz[iqz - 1 - oqz_x] = 0.f;
                     p.qz[iqz - 1] = 0.f;
-                    p.qz[iqz - sqz_x] = 0.f;
+                    p.qz[iqz - oqz_x] = 0.f;
                     const float q010 = -z0 * p.leny;
-                    p.qx[iqx - 1 - sqx_z] = 0.f;
-                    p.qx[iqx - sqx_z] = q010;
+                    p.qx[iqx - 1 - oqx_z] = 0.f;
+                    p.qx[iqx - oqx_z] = q010;
                     p.qx[iqx - 1] = y0 * p.lenz;
                     lx = q010 + vy * p.lenz;
-                    p.qy[iqy - sqy_x - sqy_z] = 0.f;
-                    p.qy[iqy - sqy_z] = 0.f;
-                    p.qy[iqy - sqy_x] = -x0 * p.lenz;
+                    p.qy[iqy - oqy_x - oqy_z] = 0.f;
+                    p.qy[iqy - oqy_z] = 0.f;
+                    p.qy[iqy - oqy_x] = -x0 * p.lenz;
                     ly = -vx * p.lenz;
                 }
             } else if (y > 0 && z > 0 && x == 0) {
@@ -237,8 +252,8 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
                 const float szByBz = sz * ip0x * ip1y * ip0z;
                 const float mx = 1.f / (sy * syByBz + sz * szByBz + eps);
                 lx = (vy * szByBz - vz * syByBz) * mx;
-                p.qz[iqz - sqz_x] = 0.f;
-                p.qy[iqy - sqy_x] = 0.f;
+                p.qz[iqz - oqz_x] = 0.f;
+                p.qy[iqy - oqy_x] = 0.f;
             } else if (x > 0 && z > 0 && y == 0) {
                 const float sxBxBz = sx * ip0x * ip0y * ip1z;
                 const float szBxBz = sz * ip1x * ip0y * ip0z;
@@ -251,36 +266,36 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
                 const float syBxBy = sy * ip1x * ip0y * ip0z;
                 const float mz = 1.f / (sx * sxBxBy + sy * syBxBy + eps);
                 lz = (vx * syBxBy - vy * sxBxBy) * mz;
-                p.qx[iqx - sqx_z] = 0.f;
-                p.qy[iqy - sqy_z] = 0.f;
+                p.qx[iqx - oqx_z] = 0.f;
+                p.qy[iqy - oqy_z] = 0.f;
             } else if (y == 0 && x > 0 && z == 0) {
-                p.qy[iqy - sqy_z] = 0.f;
+                p.qy[iqy - oqy_z] = 0.f;
                 p.qz[iqz - 1] = 0.f;
                 p.qx[iqx - 1] = 0.f;
-                p.qx[iqx - sqx_z - 1] = 0.f;
-                p.qx[iqx - sqx_z] = 0.f;
+                p.qx[iqx - oqx_z - 1] = 0.f;
+                p.qx[iqx - oqx_z] = 0.f;
             } else if (y > 0 && x == 0 && z == 0) {
-                p.qx[iqx - sqx_z] = 0.f;
-                p.qz[iqz - sqz_x] = 0.f;
-                p.qy[iqy - sqy_x - sqy_z] = 0.f;
-                p.qy[iqy - sqy_z] = 0.f;
-                p.qy[iqy - sqy_x] = 0.f;
+                p.qx[iqx - oqx_z] = 0.f;
+                p.qz[iqz - oqz_x] = 0.f;
+                p.qy[iqy - oqy_x - oqy_z] = 0.f;
+                p.qy[iqy - oqy_z] = 0.f;
+                p.qy[iqy - oqy_x] = 0.f;
             } else if (y == 0 && x == 0 && z > 0) {
                 p.qx[iqx - 1] = 0.f;
-                p.qy[iqy - sqy_x] = 0.f;
-                p.qz[iqz - sqz_x - 1] = 0.f;
-                p.qz[iqz - sqz_x] = 0.f;
+                p.qy[iqy - oqy_x] = 0.f;
+                p.qz[iqz - oqz_x - 1] = 0.f;
+                p.qz[iqz - oqz_x] = 0.f;
                 p.qz[iqz - 1] = 0.f;
             } else {
-                p.qz[iqz - 1 - sqz_x] = 0.f;
+                p.qz[iqz - 1 - oqz_x] = 0.f;
                 p.qz[iqz - 1] = 0.f;
-                p.qz[iqz - sqz_x] = 0.f;
-                p.qx[iqx - 1 - sqx_z] = 0.f;
-                p.qx[iqx - sqx_z] = 0.f;
+                p.qz[iqz - oqz_x] = 0.f;
+                p.qx[iqx - 1 - oqx_z] = 0.f;
+                p.qx[iqx - oqx_z] = 0.f;
                 p.qx[iqx - 1] = 0.f;
-                p.qy[iqy - sqy_x - sqy_z] = 0.f;
-                p.qy[iqy - sqy_z] = 0.f;
-                p.qy[iqy - sqy_x] = 0.f;
+                p.qy[iqy - oqy_x - oqy_z] = 0.f;
+                p.qy[iqy - oqy_z] = 0.f;
+                p.qy[iqy - oqy_x] = 0.f;
             }
         }
         p.qx[iqx] = lx;
@@ -297,8 +312,7 @@ __global__ void __launch_bounds__(256) project3d_kernel(Proj3Args p) {
                 p.zo[izv] = sx * ly - sy * lx;
             }
         }
-        ixv += sxv_z; iyv += syv_z; izv += szv_z;
-        iqx += sqx_z; iqy += sqy_z; iqz += sqz_z;
+        ixv += sxv_z; iyv += syv_z; iqz += sqz_z;
     }
 }
 
@@ -448,6 +462,7 @@ struct whhd_project3d_s {
     double len[3];          // domain lengths nx dx, ny dy, nz dz
     float* coef = nullptr;  // 3 axes x 3 rows x (n+1)
     whhd::AxisCoef cx, cy, cz;
+    whhd::AxisCoef cx_il, cz_il;  // rows in interleaved order
 };
 
 struct whhd_project2d_s {
@@ -481,11 +496,26 @@ int project3d_create(int nx, int ny, int nz, double dx, double dy, double dz, in
     if ((st = axis_coef(rx, nx, dx, wt, bc, true)) != WHHD_OK) return st;
     if ((st = axis_coef(ry, ny, dy, wt, bc, true)) != WHHD_OK) return st;
     if ((st = axis_coef(rz, nz, dz, wt, bc, true)) != WHHD_OK) return st;
+    // the x and z rows once more in interleaved order
+    auto interleave = [](const std::vector<float>& r, int n) {
+        std::vector<float> o(r);
+        const int lev = bitlen(n) - 1, len = n + 1;
+        for (int c = 0; c < n; ++c) {
+            int pos = c << (lev - 2);
+            if (c >= 4) {
+                const int l = bitlen(c) - 1;
+                pos = (2 * (c - (1 << l)) + 1) << (lev - 1 - l);
+            }
+            for (int k = 0; k < 3; ++k) o[k * len + pos] = r[k * len + c];
+        }
+        return o;
+    };
+    const std::vector<float> rxi = interleave(rx, nx), rzi = interleave(rz, nz);
     auto* h = new whhd_project3d_s;
     h->nx = nx; h->ny = ny; h->nz = nz;
     h->bc = bc;
     h->len[0] = nx * dx; h->len[1] = ny * dy; h->len[2] = nz * dz;
-    const size_t tot = rx.size() + ry.size() + rz.size();
+    const size_t tot = rx.size() + ry.size() + rz.size() + rxi.size() + rzi.size();
     if (hipMalloc(&h->coef, tot * sizeof(float)) != hipSuccess) {
         delete h;
         return fail(WHHD_OOM, "project3d: coefficient allocation failed");
@@ -494,6 +524,8 @@ int project3d_create(int nx, int ny, int nz, double dx, double dy, double dz, in
     all.insert(all.end(), rx.begin(), rx.end());
     all.insert(all.end(), ry.begin(), ry.end());
     all.insert(all.end(), rz.begin(), rz.end());
+    all.insert(all.end(), rxi.begin(), rxi.end());
+    all.insert(all.end(), rzi.begin(), rzi.end());
     hipError_t e = hipMemcpy(h->coef, all.data(), tot * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         hipFree(h->coef);
@@ -506,25 +538,30 @@ int project3d_create(int nx, int ny, int nz, double dx, double dy, double dz, in
     h->cy = {b, b + (ny + 1), b + 2 * (ny + 1)};
     b += 3 * (ny + 1);
     h->cz = {b, b + (nz + 1), b + 2 * (nz + 1)};
+    b += 3 * (nz + 1);
+    h->cx_il = {b, b + (nx + 1), b + 2 * (nx + 1)};
+    b += 3 * (nx + 1);
+    h->cz_il = {b, b + (nz + 1), b + 2 * (nz + 1)};
     *out = h;
     return WHHD_OK;
 }
 
 template <int ZB>
-static void launch_project3d(const Proj3Args& a, int nb, bool wide, hipStream_t st) {
+static void launch_project3d(const Proj3Args& a, int nb, bool wide, bool il, hipStream_t st) {
     // a workgroup spans up to 256 consecutive y of 256 / that many rows, so the
     // potentials' rows (ny + 1 floats, not 128-byte aligned) are written by one
     // workgroup each and few cache lines are shared between workgroups
     const int yb = a.ny >= 256 ? 256 : (a.ny >= 128 ? 128 : 64);
     dim3 block(yb, 256 / yb, 1);
     dim3 grid((a.ny + yb - 1) / yb, (a.nx + block.y - 1) / block.y, (unsigned)(a.zblocks * nb));
-    if (!wide) hipLaunchKernelGGL((project3d_kernel<int, ZB>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((project3d_kernel<int64_t, ZB>), grid, block, 0, st, a);
+    if (il) hipLaunchKernelGGL((project3d_kernel<int, ZB, true>), grid, block, 0, st, a);
+    else if (!wide) hipLaunchKernelGGL((project3d_kernel<int, ZB, false>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((project3d_kernel<int64_t, ZB, false>), grid, block, 0, st, a);
 }
 
 int project3d_run(const whhd_project3d_s* h, float* qx, float* qy, float* qz, float* xo, float* yo,
                   float* zo, const float* xv, const float* yv, const float* zv, hipStream_t st,
-                  int nb, int zb) {
+                  int nb, int zb, bool il) {
     if (!h || !qx || !qy || !qz || !xv || !yv || !zv)
         return fail(WHHD_INVALID_ARG, "project3d_run: null argument");
     if ((xo || yo || zo) && !(xo && yo && zo))
@@ -534,7 +571,7 @@ int project3d_run(const whhd_project3d_s* h, float* qx, float* qy, float* qz, fl
         return fail(WHHD_INVALID_ARG, "project3d_run: z block must be 1, 2, 4 or 8");
     const int64_t X = h->nx, Y = h->ny, Z = h->nz;
     Proj3Args a{qx, qy, qz, xo, yo, zo, xv, yv, zv, h->cx, h->cy, h->cz, h->nx, h->ny, h->nz,
-                (h->nz + zb - 1) / zb,
+                (h->nz + zb - 1) / zb, h->nx / 4, h->nz / 4,
                 {(X + 1) * Y * Z, X * (Y + 1) * Z, X * Y * (Z + 1)},
                 {X * (Y + 1) * (Z + 1), (X + 1) * Y * (Z + 1), (X + 1) * (Y + 1) * Z},
                 h->bc == 'n',
@@ -543,11 +580,16 @@ int project3d_run(const whhd_project3d_s* h, float* qx, float* qy, float* qz, fl
     if (nb < 1 || (int64_t)a.zblocks * nb > 65535)
         return fail(WHHD_INVALID_ARG, "project3d_run: batch too large for one launch");
     const bool wide = (X + 1) * (Y + 1) * (Z + 1) >= ((int64_t)1 << 31);
+    if (il && wide) return fail(WHHD_INVALID_ARG, "project3d_run: interleaved arrays of 2^31 elements");
+    if (il) {
+        a.cx = h->cx_il;
+        a.cz = h->cz_il;
+    }
     switch (zb) {
-    case 1: launch_project3d<1>(a, nb, wide, st); break;
-    case 2: launch_project3d<2>(a, nb, wide, st); break;
-    case 4: launch_project3d<4>(a, nb, wide, st); break;
-    default: launch_project3d<8>(a, nb, wide, st); break;
+    case 1: launch_project3d<1>(a, nb, wide, il, st); break;
+    case 2: launch_project3d<2>(a, nb, wide, il, st); break;
+    case 4: launch_project3d<4>(a, nb, wide, il, st); break;
+    default: launch_project3d<8>(a, nb, wide, il, st); break;
     }
     set_last_kernel("project3d_kernel");
     hipError_t e = hipGetLastError();
@@ -635,7 +677,7 @@ WHHD_API int whhd_project3d_run(whhd_project3d_t h, float* qx, float* qy, float*
                                 float* xv_out, float* yv_out, float* zv_out, const float* xv,
                                 const float* yv, const float* zv, void* stream) {
     return whhd::project3d_run(h, qx, qy, qz, xv_out, yv_out, zv_out, xv, yv, zv,
-                               (hipStream_t)stream, 1, 0);
+                               (hipStream_t)stream, 1, 0, false);
 }
 
 WHHD_API void whhd_project3d_destroy(whhd_project3d_t h) {

@@ -10,8 +10,14 @@
 // potential sizes, allocated at create: passes run out of place) and enqueues
 // everything on the caller's stream without synchronizing, so a solve can be
 // captured in a HIP graph.
+//
+// The x and z passes keep every coefficient at the position of the sample it
+// replaces (interleaved order), so that only the first forward pass writes
+// another array than it reads; the projection takes its coefficient rows in
+// that order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 
 #include "whhd_internal.h"
@@ -22,7 +28,7 @@ struct whhd_project2d_s;
 namespace whhd {
 int project3d_create(int, int, int, double, double, double, int, char, whhd_project3d_s**);
 int project3d_run(const whhd_project3d_s*, float*, float*, float*, float*, float*, float*,
-                  const float*, const float*, const float*, hipStream_t, int nb, int zb);
+                  const float*, const float*, const float*, hipStream_t, int nb, int zb, bool il);
 int project2d_create(int, int, double, double, int, char, whhd_project2d_s**);
 int project2d_run(const whhd_project2d_s*, float*, const float*, const float*, hipStream_t);
 }  // namespace whhd
@@ -90,77 +96,123 @@ __global__ void cut_kernel(float* qx, float* qy, float* qz, int nx, int ny, int 
     if (zz && iqz >= 0 && iqz < nqz) qz[iqz] = 0.f;
 }
 
-// Three line passes of one array: forward y, x, z; inverse z, y, x.  The
+// Three line passes of each array: forward y, x, z; inverse z, y, x.  The
 // separable transforms commute, so the order changes only FP32 rounding; the
 // orders are the fastest of those measured at 256^3 (forward y, x, z against
 // x, y, z: 0.697 vs 0.705 ms; inverse z, y, x against x, y, z: 0.695 vs
 // 0.698 ms).  The line-parallel kernels read and write different arrays, so
-// the passes ping-pong: in -> out -> scratch -> out.  `scratch` may be `in`
-// (consumed by the first pass) but not `out`.
+// the passes of the standard order ping-pong: in -> out -> scratch -> out.
+// `scratch` may be `in` (consumed by the first pass) but not `out`.
 struct Pass {
     char bc;
     int wt;
 };
-// Stage labels for the trace: "<fwd|inv> <array> <axis>".
-static void mark(StageTrace* tr, hipStream_t s, bool fwd, const char* arr, char axis) {
-    if (!tr || tr->cur < 0) return;
-    char lab[32];
-    std::snprintf(lab, sizeof(lab), "%s %s %c", fwd ? "fwd" : "inv", arr, axis);
-    tr->mark(s, lab);
-}
-static int three_pass(const float* in, float* scratch, size_t scratch_elems, float* out, int nx,
-                      int ny, int nz, const int lv[3], Pass px, Pass py, Pass pz, bool fwd,
-                      hipStream_t s, const whhd_recover3d_s* h, const char* arr) {
-    if ((size_t)nx * ny * nz > scratch_elems)
-        return fail(WHHD_INVALID_ARG, "recover3d: scratch smaller than the array a pass writes");
-    StageTrace* tr = const_cast<StageTrace*>(&h->trace);
-    const LineBatch b{h->nb, (int64_t)nx * ny * nz, h->lp_waves};
-    const LineBatch by{h->nb, (int64_t)nx * ny * nz, h->lp_waves_y};
-    if (fwd) {
-        TRY(transform_lines<float>(out, in, nx, ny, nz, lv[1], 'y', py.bc, py.wt, fwd, s, nullptr, &by));
-        mark(tr, s, fwd, arr, 'y');
-        TRY(transform_lines<float>(scratch, out, nx, ny, nz, lv[0], 'x', px.bc, px.wt, fwd, s, nullptr, &b));
-        mark(tr, s, fwd, arr, 'x');
-        TRY(transform_lines<float>(out, scratch, nx, ny, nz, lv[2], 'z', pz.bc, pz.wt, fwd, s, nullptr, &b));
-        mark(tr, s, fwd, arr, 'z');
-        return WHHD_OK;
-    }
-    TRY(transform_lines<float>(out, in, nx, ny, nz, lv[2], 'z', pz.bc, pz.wt, fwd, s, nullptr, &b));
-    mark(tr, s, fwd, arr, 'z');
-    TRY(transform_lines<float>(scratch, out, nx, ny, nz, lv[1], 'y', py.bc, py.wt, fwd, s, nullptr, &by));
-    mark(tr, s, fwd, arr, 'y');
-    TRY(transform_lines<float>(out, scratch, nx, ny, nz, lv[0], 'x', px.bc, px.wt, fwd, s, nullptr, &b));
-    mark(tr, s, fwd, arr, 'x');
-    return WHHD_OK;
-}
+struct Chain {
+    const float* in;
+    float* scratch;
+    size_t scratch_elems;  // elements per problem of scratch
+    float* out;
+    int nx, ny, nz;
+    Pass p[3];  // x, y, z
+    const char* name;
+};
 
 // Velocity component c (0: xv, 1: yv, 2: zv): its own axis uses the divergence
 // wavelet, the others the curl wavelet.
-static int vel_pass(whhd_recover3d_s* h, int c, const float* in, float* scratch, size_t cap,
-                    float* out, bool fwd, hipStream_t s) {
+static Chain vel_chain(const whhd_recover3d_s* h, int c, const float* in, float* scratch, size_t cap,
+                       float* out) {
+    static const char* names[3] = {"xv", "yv", "zv"};
     const Pass C{h->bc, h->wc}, D{h->bd, h->wd};
-    const int lv[3] = {h->lx, h->ly, h->lz};
-    const int X = h->nx, Y = h->ny, Z = h->nz;
-    switch (c) {
-    case 0: return three_pass(in, scratch, cap, out, X + 1, Y, Z, lv, D, C, C, fwd, s, h, "xv");
-    case 1: return three_pass(in, scratch, cap, out, X, Y + 1, Z, lv, C, D, C, fwd, s, h, "yv");
-    default: return three_pass(in, scratch, cap, out, X, Y, Z + 1, lv, C, C, D, fwd, s, h, "zv");
-    }
+    return Chain{in, scratch, cap, out, h->nx + (c == 0), h->ny + (c == 1), h->nz + (c == 2),
+                 {c == 0 ? D : C, c == 1 ? D : C, c == 2 ? D : C}, names[c]};
 }
 
 // Potential component c (0: qx, 1: qy, 2: qz): its own axis uses the curl
 // wavelet, the others the divergence wavelet.
-static int pot_pass(whhd_recover3d_s* h, int c, const float* in, float* scratch, size_t cap,
-                    float* out, bool fwd, hipStream_t s) {
+static Chain pot_chain(const whhd_recover3d_s* h, int c, const float* in, float* scratch, size_t cap,
+                       float* out) {
+    static const char* names[3] = {"qx", "qy", "qz"};
     const Pass C{h->bc, h->wc}, D{h->bd, h->wd};
-    const int lv[3] = {h->lx, h->ly, h->lz};
-    const int X = h->nx, Y = h->ny, Z = h->nz;
-    switch (c) {
-    case 0: return three_pass(in, scratch, cap, out, X, Y + 1, Z + 1, lv, C, D, D, fwd, s, h, "qx");
-    case 1: return three_pass(in, scratch, cap, out, X + 1, Y, Z + 1, lv, D, C, D, fwd, s, h, "qy");
-    default: return three_pass(in, scratch, cap, out, X + 1, Y + 1, Z, lv, D, D, C, fwd, s, h, "qz");
-    }
+    return Chain{in, scratch, cap, out, h->nx + (c != 0), h->ny + (c != 1), h->nz + (c != 2),
+                 {c == 0 ? C : D, c == 1 ? C : D, c == 2 ? C : D}, names[c]};
 }
+
+// Stage label "<fwd|inv> <array> <axis>" for the trace.
+static void mark(const whhd_recover3d_s* h, hipStream_t s, bool fwd, const char* arr, int a) {
+    StageTrace* tr = const_cast<StageTrace*>(&h->trace);
+    if (tr->cur < 0) return;
+    char lab[32];
+    std::snprintf(lab, sizeof(lab), "%s %s %c", fwd ? "fwd" : "inv", arr, "xyz"[a]);
+    tr->mark(s, lab);
+}
+
+constexpr int kOrder[2][3] = {{2, 1, 0}, {1, 0, 2}};  // inverse, forward
+
+// The three passes of one array in the standard coefficient order, ping-pong.
+static int run_chain(const whhd_recover3d_s* h, const Chain& c, bool fwd, hipStream_t s) {
+    if ((size_t)c.nx * c.ny * c.nz > c.scratch_elems)
+        return fail(WHHD_INVALID_ARG, "recover3d: scratch smaller than the array a pass writes");
+    const int lv[3] = {h->lx, h->ly, h->lz};
+    const float* src[3] = {c.in, c.out, c.scratch};
+    float* dst[3] = {c.out, c.scratch, c.out};
+    for (int i = 0; i < 3; ++i) {
+        const int a = kOrder[fwd][i];
+        const LineBatch b{h->nb, (int64_t)c.nx * c.ny * c.nz, a == 1 ? h->lp_waves_y : h->lp_waves};
+        TRY(transform_lines<float>(dst[i], src[i], c.nx, c.ny, c.nz, lv[a], "xyz"[a], c.p[a].bc, c.p[a].wt,
+                                   fwd, s, nullptr, &b));
+        mark(h, s, fwd, c.name, a);
+    }
+    return WHHD_OK;
+}
+
+// One pass of n arrays along axis a, problems p0 .. p0 + nb - 1; the x and z
+// passes in interleaved order.  dst may be src except in the forward y pass.
+static int in_place_pass(const whhd_recover3d_s* h, const Chain* ch, int n, int a,
+                         const float* const* src, float* const* dst, int p0, int nb, bool fwd,
+                         hipStream_t s) {
+    const int lv[3] = {h->lx, h->ly, h->lz};
+    const int waves = a == 1 ? h->lp_waves_y : h->lp_waves;
+    LineJob jobs[3];
+    for (int k = 0; k < n; ++k) {
+        const Chain& c = ch[k];
+        const int64_t size = (int64_t)c.nx * c.ny * c.nz;
+        jobs[k] = LineJob{dst[k] + p0 * size, src[k] + p0 * size, c.nx, c.ny, c.nz, c.p[a].bc, c.p[a].wt,
+                          size, a != 1 || !fwd};
+    }
+    const int st = lp_transform(jobs, n, lv[a], "xyz"[a], fwd, a != 1, s, waves, nb);
+    if (st != -1) return st;
+    if (a != 1) return fail(WHHD_INVALID_ARG, "recover3d: no interleaved pass");
+    for (int k = 0; k < n; ++k) {  // y lines outside the line-parallel kernels' lengths
+        const LineJob& j = jobs[k];
+        const LineBatch b{nb, j.stride, waves};
+        TRY(transform_lines<float>(j.dst, j.src, j.nx, j.ny, j.nz, lv[a], 'y', j.bc, j.wt, fwd, s, nullptr, &b));
+    }
+    return WHHD_OK;
+}
+
+// The three passes of n arrays, pass by pass over all of them.
+static int in_place_passes(const whhd_recover3d_s* h, const Chain* ch, int n, const float* const* in,
+                           float* const* out, int p0, int nb, bool fwd, hipStream_t s) {
+    const float* same[3];
+    for (int k = 0; k < n; ++k) same[k] = out[k];
+    for (int i = 0; i < 3; ++i) {
+        const int a = kOrder[fwd][i];
+        TRY(in_place_pass(h, ch, n, a, i == 0 ? in : same, out, p0, nb, fwd, s));
+        if (n == 1) mark(h, s, fwd, ch[0].name, a);
+    }
+    return WHHD_OK;
+}
+
+// Arrays up to this size (of as many problems of a batch as fit it) are solved
+// with the three components of a pass in one launch, larger ones one after the
+// other, like a traced solve, which times every array's pass.  Seven launches
+// instead of 19 (32^3 72 -> 30 us, 128^3 187 -> 83), three times the wavefronts
+// per launch, and in place the three arrays are the whole working set: up to 67
+// MB each (256^3) it fits the 256 MB Infinity Cache.  256^3: 660 us (out of
+// place, one by one), 627 (in place, one by one), 560 (in place, together);
+// 64 grids of 32^3..128^3 in groups of 17, 34, 68 and 1000 MB: 1.90, 1.90, 1.87
+// and 2.09 ms.
+constexpr int64_t kMergeBytes = 68ll << 20;
 
 // Scratch of a recovery handle, elements per problem: tmp[c] holds velocity
 // component c; sq[c] holds potential component c's coefficients and the
@@ -218,6 +270,58 @@ int recover3d_create(int nx, int ny, int nz, double dx, double dy, double dz, ch
     return WHHD_OK;
 }
 
+// A solve in the standard coefficient order, array by array and out of place:
+// lengths, wavelets or kernel modes without interleaved passes.
+static int solve_chains(const whhd_recover3d_s* h, float* const* q, float* const* vo,
+                        const float* const* v, bool vout, hipStream_t s) {
+    float* const* t = h->tmp;
+    float* const* S = h->sq;
+    const size_t* cap = h->sq_elems;
+    for (int c = 0; c < 3; ++c) TRY(run_chain(h, vel_chain(h, c, v[c], S[c], cap[c], t[c]), true, s));
+    // q coefficients land in the scratch; with v_out, s x q overwrites the
+    // transformed velocity in place at the projected coefficients
+    float* none[3] = {nullptr, nullptr, nullptr};
+    float* const* o = vout ? t : none;
+    TRY(project3d_run(h->proj, S[0], S[1], S[2], o[0], o[1], o[2], t[0], t[1], t[2], s, h->nb, h->proj_zb,
+                      false));
+    const_cast<StageTrace*>(&h->trace)->mark(s, "project");
+    for (int c = 0; c < 3; ++c) TRY(run_chain(h, pot_chain(h, c, S[c], S[c], cap[c], q[c]), false, s));
+    if (vout)
+        for (int c = 0; c < 3; ++c) TRY(run_chain(h, vel_chain(h, c, t[c], S[c], cap[c], vo[c]), false, s));
+    return WHHD_OK;
+}
+
+// Problems p0 .. p0 + nb - 1 of a solve by interleaved passes: velocity -> tmp
+// (y), then every pass in place on tmp and, after the projection, on q.
+static int solve_in_place(const whhd_recover3d_s* h, float* const* q, float* const* vo,
+                          const float* const* v, bool vout, int p0, int nb, int at_once, hipStream_t s) {
+    float* const* t = h->tmp;
+    const float* const tc[3] = {t[0], t[1], t[2]};
+    const float* const qc[3] = {q[0], q[1], q[2]};
+    Chain V[3], P[3];
+    for (int c = 0; c < 3; ++c) {
+        V[c] = vel_chain(h, c, nullptr, nullptr, 0, nullptr);
+        P[c] = pot_chain(h, c, nullptr, nullptr, 0, nullptr);
+    }
+    for (int c = 0; c < 3; c += at_once) TRY(in_place_passes(h, V + c, at_once, v + c, t + c, p0, nb, true, s));
+    float *pt[3], *pq[3];
+    for (int c = 0; c < 3; ++c) {
+        pt[c] = t[c] + p0 * (int64_t)V[c].nx * V[c].ny * V[c].nz;
+        pq[c] = q[c] + p0 * (int64_t)P[c].nx * P[c].ny * P[c].nz;
+    }
+    // with v_out, s x q overwrites the transformed velocity in place
+    float* none[3] = {nullptr, nullptr, nullptr};
+    float* const* o = vout ? pt : none;
+    TRY(project3d_run(h->proj, pq[0], pq[1], pq[2], o[0], o[1], o[2], pt[0], pt[1], pt[2], s, nb, h->proj_zb,
+                      true));
+    const_cast<StageTrace*>(&h->trace)->mark(s, "project");
+    for (int c = 0; c < 3; c += at_once) TRY(in_place_passes(h, P + c, at_once, qc + c, q + c, p0, nb, false, s));
+    if (vout)
+        for (int c = 0; c < 3; c += at_once)
+            TRY(in_place_passes(h, V + c, at_once, tc + c, vo + c, p0, nb, false, s));
+    return WHHD_OK;
+}
+
 int recover3d_solve(whhd_recover3d_s* h, float* qx, float* qy, float* qz, float* xo, float* yo,
                     float* zo, const float* xv, const float* yv, const float* zv, hipStream_t s) {
     if (!h || !qx || !qy || !qz || !xv || !yv || !zv)
@@ -225,26 +329,22 @@ int recover3d_solve(whhd_recover3d_s* h, float* qx, float* qy, float* qz, float*
     const bool vout = xo || yo || zo;
     if (vout && !(xo && yo && zo))
         return fail(WHHD_INVALID_ARG, "recover3d_solve_proj: all three v_out arrays are needed");
-    float* const* t = h->tmp;
-    float* const* S = h->sq;
     const float* v[3] = {xv, yv, zv};
     float* q[3] = {qx, qy, qz};
     float* vo[3] = {xo, yo, zo};
     h->trace.solve_start(s);
-    const size_t* cap = h->sq_elems;
-    for (int c = 0; c < 3; ++c) TRY(vel_pass(h, c, v[c], S[c], cap[c], t[c], true, s));
-    // q coefficients land in the scratch; with v_out, s x q overwrites the
-    // transformed velocity in place at the projected coefficients
-    if (vout)
-        TRY(project3d_run(h->proj, S[0], S[1], S[2], t[0], t[1], t[2], t[0], t[1], t[2], s, h->nb,
-                          h->proj_zb));
-    else
-        TRY(project3d_run(h->proj, S[0], S[1], S[2], nullptr, nullptr, nullptr, t[0], t[1], t[2], s,
-                          h->nb, h->proj_zb));
-    h->trace.mark(s, "project");
-    for (int c = 0; c < 3; ++c) TRY(pot_pass(h, c, S[c], S[c], cap[c], q[c], false, s));
-    if (vout)
-        for (int c = 0; c < 3; ++c) TRY(vel_pass(h, c, t[c], S[c], cap[c], vo[c], false, s));
+    const int64_t X = h->nx + 1, Y = h->ny + 1, Z = h->nz + 1;
+    if (g_line_kernel_mode.load() != 0 || X * Y * Z >= (int64_t)1 << 29 ||
+        !lp_interleaves(h->wc, h->bc, h->wd, h->bd, h->lx) ||
+        !lp_interleaves(h->wc, h->bc, h->wd, h->bd, h->lz)) {
+        TRY(solve_chains(h, q, vo, v, vout, s));
+    } else {
+        const int64_t bytes = (int64_t)h->nx * h->ny * h->nz * (int64_t)sizeof(float);
+        const bool one = h->trace.cur >= 0 || bytes > kMergeBytes;
+        const int per = h->trace.cur >= 0 ? h->nb : (int)std::max<int64_t>(1, kMergeBytes / bytes);
+        for (int p0 = 0; p0 < h->nb; p0 += per)
+            TRY(solve_in_place(h, q, vo, v, vout, p0, std::min(per, h->nb - p0), one ? 1 : 3, s));
+    }
     h->trace.solve_end();
     return WHHD_OK;
 }
@@ -274,7 +374,7 @@ int recover3d_cut(whhd_recover3d_s* h, float* ox, float* oy, float* oz, const fl
     const size_t pot_e[3] = {(size_t)h->nx * (h->ny + 1) * (h->nz + 1),
                              (size_t)(h->nx + 1) * h->ny * (h->nz + 1),
                              (size_t)(h->nx + 1) * (h->ny + 1) * h->nz};
-    for (int c = 0; c < 3; ++c) TRY(pot_pass(h, c, q[c], o[c], pot_e[c], S[c], true, s));
+    for (int c = 0; c < 3; ++c) TRY(run_chain(h, pot_chain(h, c, q[c], o[c], pot_e[c], S[c]), true, s));
     dim3 block(64, 4, 1);
     dim3 grid((h->ny + 1 + 63) / 64, (h->nx + 1 + 3) / 4, h->nz + 1);
     hipLaunchKernelGGL(cut_kernel, grid, block, 0, s, S[0], S[1], S[2], h->nx, h->ny, h->nz, h->lx,
@@ -283,7 +383,7 @@ int recover3d_cut(whhd_recover3d_s* h, float* ox, float* oy, float* oz, const fl
     if (e != hipSuccess) return hip_fail(e, "cut kernel");
     set_last_kernel("cut_kernel");
     h->trace.mark(s, "cut");
-    for (int c = 0; c < 3; ++c) TRY(pot_pass(h, c, S[c], S[c], h->sq_elems[c], o[c], false, s));
+    for (int c = 0; c < 3; ++c) TRY(run_chain(h, pot_chain(h, c, S[c], S[c], h->sq_elems[c], o[c]), false, s));
     h->trace.solve_end();
     return WHHD_OK;
 }

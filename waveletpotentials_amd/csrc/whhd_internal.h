@@ -67,10 +67,26 @@ int transform_lines(T* dst, const T* src, int nx, int ny, int nz, int levels, ch
                     int wt, bool fwd, hipStream_t stream, const TileConfig* cfg = nullptr,
                     const LineBatch* batch = nullptr);
 
-// Line-parallel transform (dst != src, curl CDF3.7 'n' / divergence CDF4.6 'd',
-// 2^5..2^8 samples); returns -1 when no such kernel applies.
-int lp_transform(float* dst, const float* src, int nx, int ny, int nz, int levels, char axis,
-                 char bc, int wt, bool fwd, hipStream_t stream, const LineBatch& b);
+// One array's line pass: dst = transform of src along the launch's axis;
+// problems of a batch `stride` elements apart.
+struct LineJob {
+    float* dst;
+    const float* src;
+    int nx, ny, nz;
+    char bc;
+    int wt;
+    int64_t stride;
+    bool in_place = false;  // dst may equal src
+};
+
+// Line-parallel transform of 1..3 arrays along one axis in one launch (the
+// wavelets of one recovery pair, 2^3..2^8 samples); returns -1 when no such
+// kernel applies.  Interleaved (x and z axes): every coefficient at the position
+// of the sample it replaces, see line_parallel.h.  dst may equal src (in_place)
+// in the inverse and in either direction interleaved.
+int lp_transform(const LineJob* jobs, int njobs, int levels, char axis, bool fwd, bool interleaved,
+                 hipStream_t stream, int waves, int nb);
+bool lp_interleaves(int wt_curl, char bc_curl, int wt_div, char bc_div, int levels);
 
 // Recovery driver over `nb` problems of equal extents stored back to back (the
 // arrays of problem b start b * (array size) elements after the first);
