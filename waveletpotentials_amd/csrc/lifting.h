@@ -439,18 +439,18 @@ struct Wavelet {
 };
 
 // y = M x over lanes 0..M-1 (lane r gets row r); other lanes return row 0.
+// Each lane loads its own row: M loads in flight together, the same for every
+// line a wavefront lifts (selecting the row from scalar loads of the whole
+// matrix waited for four of them in turn).
 template <int M, const double* Mat, class T>
 WHHD_DEV T apply_l10(T v, int lane) {
-    const int r = lane < M ? lane : 0;
+    const double* row = Mat + (lane < M ? lane : 0) * M;
+    T coef[M];
+#pragma unroll
+    for (int c = 0; c < M; ++c) coef[c] = T(row[c]);
     T acc = T(0);
 #pragma unroll
-    for (int c = 0; c < M; ++c) {
-        T xc = lane_get(v, c);
-        T coef = T(0);
-#pragma unroll
-        for (int rr = 0; rr < M; ++rr) coef = (r == rr) ? T(Mat[rr * M + c]) : coef;
-        acc += xc * coef;
-    }
+    for (int c = 0; c < M; ++c) acc += lane_get(v, c) * coef[c];
     return acc;
 }
 

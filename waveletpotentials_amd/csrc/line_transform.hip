@@ -133,8 +133,7 @@ WHHD_DEV T* inverse_line(T* in, T* other, int n, int levels, int lane) {
 // at outer index blockIdx.y; sample i of line (y, o) sits at
 // y + o*outer_stride + i*sample_stride.
 template <class W, class T, bool FWD, bool STRIDED>
-__global__ void __launch_bounds__(256) line_tile_kernel(T* __restrict__ dst,
-                                                        const T* __restrict__ src, LineGeom g) {
+WHHD_DEV void line_tile(T* dst, const T* src, const LineGeom& g, unsigned tile_index) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* sm = reinterpret_cast<T*>(smem_raw);
     const int n = g.n;
@@ -151,11 +150,11 @@ __global__ void __launch_bounds__(256) line_tile_kernel(T* __restrict__ dst,
     int64_t tile_base;  // element offset of line 0 of the tile
     int lines_here;
     if (!STRIDED) {
-        const int64_t first = (int64_t)blockIdx.x * tile;
+        const int64_t first = (int64_t)tile_index * tile;
         lines_here = (int)min<int64_t>((int64_t)tile, g.lines - first);
         tile_base = first * n;
     } else {
-        const int y0 = blockIdx.x * tile;
+        const int y0 = tile_index * tile;
         lines_here = min(tile, g.lines - y0);
         tile_base = (int64_t)y0 + (int64_t)blockIdx.y * g.outer_stride;
     }
@@ -210,6 +209,22 @@ __global__ void __launch_bounds__(256) line_tile_kernel(T* __restrict__ dst,
     }
 }
 
+template <class W, class T, bool FWD, bool STRIDED>
+__global__ void __launch_bounds__(256) line_tile_kernel(T* __restrict__ dst,
+                                                        const T* __restrict__ src, LineGeom g) {
+    line_tile<W, T, FWD, STRIDED>(dst, src, g, blockIdx.x);
+}
+
+// Forward pass of two arrays along one axis in one launch: the first `tiles_a`
+// workgroups of a row take array a (wavelet WA), the others array b (WB).
+template <class WA, class WB, bool STRIDED>
+__global__ void __launch_bounds__(256) line_tile_pair_kernel(float* da, const float* sa, LineGeom ga,
+                                                             unsigned tiles_a, float* db,
+                                                             const float* sb, LineGeom gb) {
+    if (blockIdx.x < tiles_a) line_tile<WA, float, true, STRIDED>(da, sa, ga, blockIdx.x);
+    else line_tile<WB, float, true, STRIDED>(db, sb, gb, blockIdx.x - tiles_a);
+}
+
 // ---------------------------------------------------------------------------
 // Host-side dispatch
 // ---------------------------------------------------------------------------
@@ -228,6 +243,15 @@ static hipError_t launch_w(T* dst, const T* src, const LineGeom& g, bool fwd, bo
         else hipLaunchKernelGGL((line_tile_kernel<W, T, false, true>), grid, block, smem, stream, dst, src, g);
     }
     return hipGetLastError();
+}
+
+// Arrays of up to 4096 lines get four lines (one per wavefront) a workgroup:
+// with the larger tiles, which suit the memory system, they occupy a few CUs
+// and every wavefront lifts several lines one after the other.
+static void few_lines(TileConfig& c, int64_t lines) {
+    if (lines > 4096) return;
+    if (c.strided_tile > 4) c.strided_tile = 4;
+    if (c.contig_tile > 4) c.contig_tile = 4;
 }
 
 template <class T>
@@ -286,6 +310,7 @@ int transform_lines(T* dst, const T* src, int nx, int ny, int nz, int levels, ch
     g.levels = levels;
     g.lds_row = (n & 1) ? n : n + 1;
     TileConfig c = cfg ? *cfg : default_tile(n, sizeof(T), strided);
+    if (!cfg) few_lines(c, g.lines * (strided ? g.outer : 1));
     g.tile = strided ? c.strided_tile : c.contig_tile;
     if (g.tile <= 0) return WHHD_INVALID_ARG;
     if ((size_t)2 * g.tile * g.lds_row * sizeof(T) > kMaxLdsBytes) return WHHD_INVALID_ARG;
@@ -299,6 +324,59 @@ int transform_lines(T* dst, const T* src, int nx, int ny, int nz, int levels, ch
                   sizeof(T) == sizeof(float) ? "f32" : "f64");
     set_last_kernel(name);
     return e == hipSuccess ? WHHD_OK : hip_fail(e, "line tile kernel");
+}
+
+// Forward pass along `axis` of two 2D arrays in one launch, in place; -1 when
+// the wavelets are not a curl / divergence pair with a pair kernel or a line
+// does not fit.  Arrays of a few thousand lines: one line per wavefront, four
+// to a workgroup, so the lines spread over the chip.
+int transform_pair2d(const LineJob& a, const LineJob& b, int levels, char axis, hipStream_t stream) {
+    const LineJob* j[2] = {&a, &b};
+    LineGeom g[2];
+    unsigned tiles[2];
+    const bool strided = axis == 'x';
+    size_t smem = 0;
+    for (int k = 0; k < 2; ++k) {
+        const int n = strided ? j[k]->nx : j[k]->ny;
+        const int lines = strided ? j[k]->ny : j[k]->nx;
+        if (check_wavelet(j[k]->wt, j[k]->bc) != WHHD_OK || check_line(n, levels, j[k]->wt) != WHHD_OK) return -1;
+        g[k].n = n;
+        g[k].levels = levels;
+        g[k].lds_row = (n & 1) ? n : n + 1;
+        g[k].lines = lines;
+        g[k].sample_stride = strided ? j[k]->ny : 1;
+        TileConfig c = default_tile(n, sizeof(float), strided);
+        few_lines(c, lines);
+        g[k].tile = strided ? c.strided_tile : c.contig_tile;
+        tiles[k] = (unsigned)((lines + g[k].tile - 1) / g[k].tile);
+        const size_t need = (size_t)2 * g[k].tile * g[k].lds_row * sizeof(float);
+        if (need > kMaxLdsBytes) return -1;
+        smem = need > smem ? need : smem;
+    }
+    const dim3 grid(tiles[0] + tiles[1]), block(256);
+#define WHHD_PAIR(A, B)                                                                            \
+    do {                                                                                           \
+        if (strided)                                                                               \
+            hipLaunchKernelGGL((line_tile_pair_kernel<A, B, true>), grid, block, smem, stream,     \
+                               a.dst, a.src, g[0], tiles[0], b.dst, b.src, g[1]);                  \
+        else                                                                                       \
+            hipLaunchKernelGGL((line_tile_pair_kernel<A, B, false>), grid, block, smem, stream,    \
+                               a.dst, a.src, g[0], tiles[0], b.dst, b.src, g[1]);                  \
+    } while (0)
+    auto is = [](const LineJob& q, int wt, char bc) { return q.wt == wt && q.bc == bc; };
+    if (is(a, WT_CDF4_6, 'd') && is(b, WT_CDF3_7, 'n')) WHHD_PAIR(W_Cdf46D, W_Cdf37N);
+    else if (is(a, WT_CDF3_7, 'n') && is(b, WT_CDF4_6, 'd')) WHHD_PAIR(W_Cdf37N, W_Cdf46D);
+    else if (is(a, WT_CDF4_6, 'n') && is(b, WT_CDF3_7, 'd')) WHHD_PAIR(W_Cdf46N, W_Cdf37D);
+    else if (is(a, WT_CDF3_7, 'd') && is(b, WT_CDF4_6, 'n')) WHHD_PAIR(W_Cdf37D, W_Cdf46N);
+    else if (is(a, WT_CDF4_4, 'd') && is(b, WT_CDF3_5, 'n')) WHHD_PAIR(W_Cdf44D, W_Cdf35N);
+    else if (is(a, WT_CDF3_5, 'n') && is(b, WT_CDF4_4, 'd')) WHHD_PAIR(W_Cdf35N, W_Cdf44D);
+    else if (is(a, WT_CDF4_4, 'n') && is(b, WT_CDF3_5, 'd')) WHHD_PAIR(W_Cdf44N, W_Cdf35D);
+    else if (is(a, WT_CDF3_5, 'd') && is(b, WT_CDF4_4, 'n')) WHHD_PAIR(W_Cdf35D, W_Cdf44N);
+    else return -1;
+#undef WHHD_PAIR
+    set_last_kernel("line_tile_pair_kernel");
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? WHHD_OK : hip_fail(e, "line tile pair kernel");
 }
 
 template int transform_lines<float>(float*, const float*, int, int, int, int, char, char, int, bool,

@@ -426,10 +426,22 @@ int recover2d_solve(whhd_recover2d_s* h, float* qz, const float* xv, const float
     const int X = h->nx, Y = h->ny;
     float* tx = h->tmp[0];
     float* ty = h->tmp[1];
-    TRY(transform_lines<float>(tx, xv, X + 1, Y, 1, h->lx, 'x', h->bd, h->wd, true, s));
-    TRY(transform_lines<float>(tx, tx, X + 1, Y, 1, h->ly, 'y', h->bc, h->wc, true, s));
-    TRY(transform_lines<float>(ty, yv, X, Y + 1, 1, h->lx, 'x', h->bc, h->wc, true, s));
-    TRY(transform_lines<float>(ty, ty, X, Y + 1, 1, h->ly, 'y', h->bd, h->wd, true, s));
+    // The windowed kernels throughout: a 2D array has too few lines to fill the
+    // chip with a line per lane.
+    const LineJob ax{tx, xv, X + 1, Y, 1, h->bd, h->wd, 0}, bx{ty, yv, X, Y + 1, 1, h->bc, h->wc, 0};
+    int r = transform_pair2d(ax, bx, h->lx, 'x', s);
+    if (r == -1) {
+        TRY(transform_lines<float>(tx, xv, X + 1, Y, 1, h->lx, 'x', h->bd, h->wd, true, s));
+        r = transform_lines<float>(ty, yv, X, Y + 1, 1, h->lx, 'x', h->bc, h->wc, true, s);
+    }
+    TRY(r);
+    const LineJob ay{tx, tx, X + 1, Y, 1, h->bc, h->wc, 0}, by{ty, ty, X, Y + 1, 1, h->bd, h->wd, 0};
+    r = transform_pair2d(ay, by, h->ly, 'y', s);
+    if (r == -1) {
+        TRY(transform_lines<float>(tx, tx, X + 1, Y, 1, h->ly, 'y', h->bc, h->wc, true, s));
+        r = transform_lines<float>(ty, ty, X, Y + 1, 1, h->ly, 'y', h->bd, h->wd, true, s);
+    }
+    TRY(r);
     TRY(project2d_run(h->proj, qz, tx, ty, s));
     TRY(transform_lines<float>(qz, qz, X + 1, Y + 1, 1, h->lx, 'x', h->bd, h->wd, false, s));
     TRY(transform_lines<float>(qz, qz, X + 1, Y + 1, 1, h->ly, 'y', h->bd, h->wd, false, s));

@@ -88,6 +88,10 @@ int lp_transform(const LineJob* jobs, int njobs, int levels, char axis, bool fwd
                  hipStream_t stream, int waves, int nb);
 bool lp_interleaves(int wt_curl, char bc_curl, int wt_div, char bc_div, int levels);
 
+// Forward pass along `axis` ('x' or 'y') of two 2D arrays in one launch of the
+// windowed kernels, in place (dst == src); -1 when no pair kernel applies.
+int transform_pair2d(const LineJob& a, const LineJob& b, int levels, char axis, hipStream_t stream);
+
 // Recovery driver over `nb` problems of equal extents stored back to back (the
 // arrays of problem b start b * (array size) elements after the first);
 // recover3d_set_tiles picks the launch shapes (1/2/4 wavefronts per line-pass
