@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstdint>
 
 #include "whhd_internal.h"
 
@@ -109,33 +110,85 @@ __device__ __forceinline__ float eikonal_update(float a, float b, float c, float
 // One thread per (x, y) column walks kEikZ consecutive z cells, carrying the
 // z - 1, z and z + 1 values in registers, so every value is loaded once per
 // column walk (the in-plane neighbours come from the caches) instead of up to
-// three times.
-constexpr int kEikZ = 16;  // 4, 8 and 16 time alike at 192^3 (~20 us); 32: 30 us
-
+// three times.  A neighbour outside the grid is read on the other side instead
+// and the smaller of the two capped at 1e8: one select an axis instead of one a
+// neighbour.  Offsets are 32-bit bytes when the array allows (I).
+//
+// Tiles (64 y x 4 x x kEikZ z, a workgroup's) that cannot change are left out.
+// A relaxation is a pure function of a cell and its six neighbours, so a tile
+// whose own cells and whose six neighbour tiles did not change a bit in the last
+// relaxation does not change in this one, and both iterates already hold it.
+// chg_in[tile] says whether the last relaxation changed it (null: all did),
+// chg_out[tile] receives this one's.  The field settles outwards from the solids
+// (a cell depends on smaller neighbours only), long before the 1.5-2 max(n)
+// relaxations that a caller asks for to be sure.
+// 320 relaxations of 160x120x136: 3.59 -> 1.84 ms (2.49 with a load behind every
+// store), 384 of 192^3: 6.31 -> 3.53.
+//
+// kEikZ: 8, or 4 on grids that would give fewer than 512 workgroups (64x48x40: 4
+// 3.1 us a relaxation, 8 3.6; 160x120x136: 4 6.0, 8 5.8, 16 8.5).
+template <class I, int kEikZ>
 __global__ void __launch_bounds__(256) eikonal_kernel(float* __restrict__ dst, const float* __restrict__ src,
-                                                      int nx, int ny, int nz, float h) {
+                                                      int nx, int ny, int nz, float h,
+                                                      const uint8_t* __restrict__ chg_in,
+                                                      uint8_t* __restrict__ chg_out) {
+    const unsigned gx = gridDim.x, gy = gridDim.y;
+    const unsigned tile = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+    if (chg_in) {
+        int any = chg_in[tile];
+        if (blockIdx.x > 0) any |= chg_in[tile - 1];
+        if (blockIdx.x + 1 < gx) any |= chg_in[tile + 1];
+        if (blockIdx.y > 0) any |= chg_in[tile - gx];
+        if (blockIdx.y + 1 < gy) any |= chg_in[tile + gx];
+        if (blockIdx.z > 0) any |= chg_in[tile - gx * gy];
+        if (blockIdx.z + 1 < gridDim.z) any |= chg_in[tile + gx * gy];
+        if (!any) {
+            if (threadIdx.x == 0 && threadIdx.y == 0) chg_out[tile] = 0;
+            return;
+        }
+    }
     const int y = blockIdx.x * 64 + threadIdx.x;
     const int x = blockIdx.y * 4 + threadIdx.y;
     const int z0 = blockIdx.z * kEikZ;
-    if (y >= ny || x >= nx) return;
-    const int64_t sx = ny, sz = (int64_t)nx * ny;
-    constexpr float kFar = 1e8f;
-    int64_t i = y + x * sx + z0 * sz;
-    float below = z0 > 0 ? src[i - sz] : kFar;
-    float c = src[i];
-    const int zend = min(z0 + kEikZ, nz);
-    for (int z = z0; z < zend; ++z, i += sz) {
-        const float above = z < nz - 1 ? src[i + sz] : kFar;
-        // neighbours through clamped (always valid) indices, replaced by kFar
-        // outside the grid: no branch per load
-        const float l0 = src[i - (x > 0 ? sx : 0)], r0 = src[i + (x < nx - 1 ? sx : 0)];
-        const float d0 = src[i - (y > 0 ? 1 : 0)], u0 = src[i + (y < ny - 1 ? 1 : 0)];
-        const float l = x > 0 ? l0 : kFar, r = x < nx - 1 ? r0 : kFar;
-        const float d = y > 0 ? d0 : kFar, u = y < ny - 1 ? u0 : kFar;
-        const float upd = eikonal_update(fminf(l, r), fminf(d, u), fminf(below, above), h);
-        dst[i] = c > -1e-12f ? upd : c;
-        below = c;
-        c = above;
+    int changed = 0;
+    if (y < ny && x < nx) {
+        constexpr float kFar = 1e8f;
+        const I sx = (I)ny * 4, sz = (I)nx * ny * 4;
+        const I il = x > 0 ? -sx : (nx > 1 ? sx : 0), ir = x < nx - 1 ? sx : il;
+        const I id = y > 0 ? I(-4) : (ny > 1 ? I(4) : 0), iu = y < ny - 1 ? I(4) : id;
+        const bool bx = x == 0 || x == nx - 1, by = y == 0 || y == ny - 1;
+        auto at = [&](I o) { return *(const float*)((const char*)src + o); };
+        const I i0 = (I)y * 4 + (I)x * sx + (I)z0 * sz;
+        // every load before the first store (the iterates may alias as far as the
+        // compiler knows, and a load behind a store waits out its own latency in
+        // each cell); cells past the last plane read that plane
+        const int last = nz - 1 - z0;
+        float col[kEikZ + 2], mx[kEikZ], my[kEikZ];
+        col[0] = at(z0 > 0 ? i0 - sz : i0);
+#pragma unroll
+        for (int k = 0; k < kEikZ + 1; ++k) col[k + 1] = at(i0 + (I)min(k, last) * sz);
+#pragma unroll
+        for (int k = 0; k < kEikZ; ++k) {
+            const I i = i0 + (I)min(k, last) * sz;
+            mx[k] = fminf(at(i + il), at(i + ir));
+            my[k] = fminf(at(i + id), at(i + iu));
+        }
+        if (z0 == 0) col[0] = kFar;
+#pragma unroll
+        for (int k = 0; k < kEikZ; ++k) {
+            if (k > last) break;
+            const float above = k < last ? col[k + 2] : kFar, c = col[k + 1];
+            const float ax = bx ? fminf(nx > 1 ? mx[k] : kFar, kFar) : mx[k];
+            const float ay = by ? fminf(ny > 1 ? my[k] : kFar, kFar) : my[k];
+            const float upd = eikonal_update(ax, ay, fminf(col[k], above), h);
+            const float v = c > -1e-12f ? upd : c;
+            changed |= __float_as_int(v) != __float_as_int(c);
+            *(float*)((char*)dst + i0 + (I)k * sz) = v;
+        }
+    }
+    if (chg_out) {
+        changed = __syncthreads_or(changed);
+        if (threadIdx.x == 0 && threadIdx.y == 0) chg_out[tile] = (uint8_t)(changed != 0);
     }
 }
 
@@ -355,13 +408,34 @@ int eikonal_sweep(float* ls, float* scratch, int nx, int ny, int nz, double h, i
     if (st != WHHD_OK) return st;
     float* a = ls;
     float* b = scratch;
+    const int64_t columns = (int64_t)((ny + 63) / 64) * ((nx + 3) / 4);
+    const int zb = columns * ((nz + 7) / 8) < 512 ? 4 : 8;
+    const dim3 grid((ny + 63) / 64, (nx + 3) / 4, (nz + zb - 1) / zb);
+    const size_t tiles = (size_t)grid.x * grid.y * grid.z;
+    // two sets of tile flags from the stream's memory pool; without them (few
+    // relaxations, a stream being captured, no memory) every tile runs
+    uint8_t* flags = nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (n_iters >= 8 && hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+        hipMallocAsync((void**)&flags, 2 * tiles, s) != hipSuccess) {
+        (void)hipGetLastError();
+        flags = nullptr;
+    }
+    const bool wide = (int64_t)nx * ny * nz * 4 >= (int64_t)1 << 31;
     for (int i = 0; i < n_iters; ++i) {
-        hipLaunchKernelGGL(eikonal_kernel, dim3((ny + 63) / 64, (nx + 3) / 4, (nz + kEikZ - 1) / kEikZ),
-                           dim3(64, 4), 0, s, b, a, nx, ny, nz, (float)h);
+        const uint8_t* in = flags && i > 0 ? flags + (i & 1) * tiles : nullptr;
+        uint8_t* out = flags ? flags + (1 - (i & 1)) * tiles : nullptr;
+        if (wide)
+            hipLaunchKernelGGL((eikonal_kernel<int64_t, 8>), grid, dim3(64, 4), 0, s, b, a, nx, ny, nz, (float)h, in, out);
+        else if (zb == 8)
+            hipLaunchKernelGGL((eikonal_kernel<int, 8>), grid, dim3(64, 4), 0, s, b, a, nx, ny, nz, (float)h, in, out);
+        else
+            hipLaunchKernelGGL((eikonal_kernel<int, 4>), grid, dim3(64, 4), 0, s, b, a, nx, ny, nz, (float)h, in, out);
         float* t = a;
         a = b;
         b = t;
     }
+    if (flags) (void)hipFreeAsync(flags, s);
     set_last_kernel("eikonal_kernel");
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "eikonal kernel");
