@@ -14,6 +14,7 @@
 // matrix (an LDS-tiled kernel over 64 x 64 output tiles).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 #include <type_traits>
@@ -22,6 +23,12 @@
 #include "whhd_internal.h"
 
 namespace whhd {
+
+// dst_lines.hip
+bool dst_lines(int logm, bool contig, float* out, const float* in, int64_t lines, int64_t n_inner,
+               int64_t s_inner, int64_t s_outer, int64_t step, float c, const float* lam_q,
+               const float* lam_r, const float* lam_s, int64_t lam_div, int reps, hipStream_t s);
+
 namespace {
 
 // One thread per node column (x <= nx, y <= ny): the qx column (x < nx) and qy
@@ -110,16 +117,25 @@ __global__ void __launch_bounds__(64 * kGaugeWaves) top_gauge_kernel(T* __restri
 
 // Velocity bc 'd' bottom plane (SweepingQy_x, WaveletPotentials/cuParallelSweep3D.cu:
 // 68-85): per y, qy(x, y, 0) = sum_{x' < x} zv(x', y, 0) dx.
+// One wavefront per 64 y, sixteen loads in flight (one at a time, a serial chain of
+// memory latencies: 96 of them 25 -> 9 us).
 template <class T>
-__global__ void bottom_qy_kernel(T* __restrict__ qy, const T* __restrict__ zv, int nx,
-                                 int ny, T dx) {
+__global__ void __launch_bounds__(64) bottom_qy_kernel(T* __restrict__ qy, const T* __restrict__ zv, int nx,
+                                                       int ny, T dx) {
     const int y = blockIdx.x * blockDim.x + threadIdx.x;
     if (y >= ny) return;
     T acc = T(0);
     qy[y] = T(0);
-    for (int x = 1; x <= nx; ++x) {
-        acc += zv[y + (int64_t)(x - 1) * ny] * dx;
-        qy[y + (int64_t)x * ny] = acc;
+    for (int x = 1; x <= nx; x += 16) {
+        T v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = zv[y + (int64_t)min(x + u - 1, nx - 1) * ny];
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+            if (x + u <= nx) {
+                acc += v[u] * dx;
+                qy[y + (int64_t)(x + u) * ny] = acc;
+            }
     }
 }
 
@@ -290,6 +306,134 @@ __global__ void __launch_bounds__(256) dst_pass_kernel(T* __restrict__ out,
             const int gi = i0 + ti + r, gk = k0 + tk + c;
             if (gi < m && gk < n) out[boff + gi * si + gk * sj] = acc[r][c];
         }
+}
+
+// The same product with a line per lane, for lines of up to kStripMax samples.
+// The sine matrix folds, S(k, n - 1 - j) = (-1)^k S(k, j): output k needs only the
+// sums (even k) or differences (odd k) of samples j and n - 1 - j, half the
+// products.  A wavefront takes 64 lines and a strip of KB outputs of one parity; the
+// samples come from vector loads (coalesced along the lines on the x and z axes, from
+// the L1 along y), the strip's KB sine values per j from scalar loads: no LDS, no
+// barrier.  On short lines the tiled kernel above is a serial chain of slices, each
+// waiting out a load and two barriers; on long ones it reads less.  Poisson solve
+// (six passes), us, tiled / strips: FP64 97x81x61 145 / 79, 120^3 268 / 151; FP32 49^3
+// 75 / 48, 200x180x160 425 / 300, 300^3 2299 / 2137.
+// Table: row j < (n + 1) / 2 holds S(k, j) for even k, then odd k, each part padded
+// with zeros to whole strips; row (n - 1) / 2 of odd n, whose sample meets itself,
+// is halved.
+// With lam_s set, divides by the eigenvalue sum as DstScale describes.
+template <class T>
+constexpr int kStrip = sizeof(T) == 8 ? 8 : 16;
+template <class T>
+constexpr int kStripMax = sizeof(T) == 8 ? 256 : 320;
+template <class T>
+int strips(int outputs) { return (outputs + kStrip<T> - 1) / kStrip<T>; }
+
+template <class T>
+__global__ void __launch_bounds__(256) dst_strip_kernel(T* __restrict__ out, const T* __restrict__ in,
+                                                        const T* __restrict__ S, int n, int64_t lines, int m,
+                                                        int64_t si, int64_t sj, int64_t sb,
+                                                        const T* __restrict__ lam_q, const T* __restrict__ lam_r,
+                                                        const T* __restrict__ lam_s, int lam_div) {
+    constexpr int KB = kStrip<T>;
+    const int even = ((n + 1) / 2 + KB - 1) / KB, all = even + (n / 2 + KB - 1) / KB;
+    const int strip = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + (threadIdx.x >> 6));
+    if (strip >= all) return;
+    const bool odd = strip >= even;
+    const int k0 = odd ? 1 + 2 * (strip - even) * KB : 2 * strip * KB;  // outputs k0, k0 + 2, ...
+    const int pitch = all * KB, rows = (n + 1) / 2;
+    const uint32_t li = blockIdx.x * 64 + (threadIdx.x & 63);  // the arrays hold less than 2^31 elements
+    const bool ok = li < (uint32_t)lines;
+    const uint32_t l = ok ? li : 0, b = l / (uint32_t)m, i = l - b * (uint32_t)m;
+    const int64_t base = (int64_t)i * si + (int64_t)b * sb;
+    const T* lo = in + base;
+    const T* hi = lo + (n - 1) * sj;
+    const T* s = S + strip * KB;
+    const T sign = odd ? T(-1) : T(1);
+    T acc[KB];
+#pragma unroll
+    for (int q = 0; q < KB; ++q) acc[q] = T(0);
+    int j = 0;
+    for (; j + 4 <= rows; j += 4) {
+        T v[4], w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            v[u] = lo[(j + u) * sj];
+            w[u] = hi[-(j + u) * sj];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const T f = v[u] + sign * w[u];
+#pragma unroll
+            for (int q = 0; q < KB; ++q) acc[q] += f * s[q];
+            s += pitch;
+        }
+    }
+    for (; j < rows; ++j) {
+        const T f = lo[j * sj] + sign * hi[-j * sj];
+#pragma unroll
+        for (int q = 0; q < KB; ++q) acc[q] += f * s[q];
+        s += pitch;
+    }
+    if (!ok) return;
+    if (lam_s) {
+        const T sum = lam_q[l / (uint32_t)lam_div] + lam_r[l % (uint32_t)lam_div];
+#pragma unroll
+        for (int q = 0; q < KB; ++q)
+            if (k0 + 2 * q < n) acc[q] /= sum + lam_s[k0 + 2 * q];
+    }
+    T* dst = out + base + k0 * sj;
+#pragma unroll
+    for (int q = 0; q < KB; ++q)
+        if (k0 + 2 * q < n) dst[2 * q * sj] = acc[q];
+}
+
+// The strips of contiguous lines (the y axis) in one workgroup per 64 lines: the
+// lines are one block of memory, staged in LDS (rows of n | 1 values, so the
+// lanes' walks hit every bank once), and the outputs go back through LDS the same
+// way.  Lane by lane from memory every load and store touches 64 lines of it: from
+// 2^20 samples this is the faster one (a 120^3 FP64 solve 169 -> 151 us, FP32 153 ->
+// 128; 49^3 37 -> 44 and 48 -> 54, where its second barrier and copy weigh more).
+template <class T>
+__global__ void __launch_bounds__(1024) dst_strip_rows_kernel(T* __restrict__ out, const T* __restrict__ in, const T* __restrict__ S,
+                                      int n, int64_t lines) {
+    extern __shared__ unsigned char dst_rows_smem[];
+    constexpr int KB = kStrip<T>;
+    const int rs = n | 1;
+    T* rows_in = (T*)dst_rows_smem;
+    T* rows_out = rows_in + 64 * rs;
+    const int64_t first = (int64_t)blockIdx.x * 64;
+    const int here = (int)min((int64_t)64, lines - first), total = here * n;
+    const T* src = in + first * n;
+    for (int e = threadIdx.x; e < total; e += blockDim.x) rows_in[e / n * rs + e % n] = src[e];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+    const int even = ((n + 1) / 2 + KB - 1) / KB, all = even + (n / 2 + KB - 1) / KB;
+    const int pitch = all * KB, rows = (n + 1) / 2;
+    const T* lo = rows_in + (lane < here ? lane : 0) * rs;
+    T* dst = rows_out + lane * rs;
+    for (int strip = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); strip < all; strip += waves) {
+        const bool odd = strip >= even;
+        const int k0 = odd ? 1 + 2 * (strip - even) * KB : 2 * strip * KB;
+        const T sign = odd ? T(-1) : T(1);
+        const T* s = S + strip * KB;
+        T acc[KB];
+#pragma unroll
+        for (int q = 0; q < KB; ++q) acc[q] = T(0);
+#pragma unroll 4
+        for (int j = 0; j < rows; ++j) {
+            const T f = lo[j] + sign * lo[n - 1 - j];
+#pragma unroll
+            for (int q = 0; q < KB; ++q) acc[q] += f * s[q];
+            s += pitch;
+        }
+#pragma unroll
+        for (int q = 0; q < KB; ++q)
+            if (k0 + 2 * q < n) dst[k0 + 2 * q] = acc[q];
+    }
+    __syncthreads();
+    T* o = out + first * n;
+    for (int e = threadIdx.x; e < total; e += blockDim.x) o[e] = rows_out[e / n * rs + e % n];
 }
 
 // ---- DST-I through a half-length complex FFT ---------------------------------
@@ -717,6 +861,15 @@ int dst_pass(const whhd_dst3d_s* h, T* out, const T* in, int a, hipStream_t s,
             else sc = DstScale{h->lam[2], h->lam[0], h->lam[1], n1};
         }
         const T c = (T)std::sqrt(2.0 / M);
+        if constexpr (!is64<T>()) {
+            // 255^3 462 -> 213 us a solve, 127^3 96 -> 60, 31^3 99 -> 20, 255x31x15 107 -> 44: faster
+            // at every size; contiguous lines need 16-byte aligned arrays
+            if (dst_lines(lm, a == 1, out, in, lines, n_inner, s_inner, s_outer, step, c,
+                          (const T*)sc.lam_q, (const T*)sc.lam_r, (const T*)sc.lam_s, sc.lam_div, reps, s)) {
+                hipError_t e = done("dst_lines_kernel");
+                return e == hipSuccess ? WHHD_OK : hip_fail(e, "dst lines kernel");
+            }
+        }
         const T* tab = (const T*)h->S[a];
 #define WHHD_DST_FFT(L) \
     case L: hipLaunchKernelGGL((dst_fft_kernel<T, L>), grid, dim3(kFftThreads), lds, s, out, in, tab, n, \
@@ -729,6 +882,25 @@ int dst_pass(const whhd_dst3d_s* h, T* out, const T* in, int a, hipStream_t s,
 #undef WHHD_DST_FFT
         hipError_t e = done("dst_fft_kernel");
         return e == hipSuccess ? WHHD_OK : hip_fail(e, "dst fft kernel");
+    }
+    if (n <= kStripMax<T>) {
+        const int64_t lines = (int64_t)m * nb;
+        const int all = strips<T>((n + 1) / 2) + strips<T>(n / 2);
+        // lines of the z pass are li = y + x n2
+        const T* const none = nullptr;
+        const size_t rows_lds = 2 * 64 * (size_t)(n | 1) * sizeof(T);
+        if (sj == 1 && rows_lds <= kMaxLdsBytes && !scale && lines * n >= 1 << 20) {
+            hipLaunchKernelGGL(dst_strip_rows_kernel<T>, dim3((unsigned)((lines + 63) / 64)),
+                               dim3(64 * std::min(all, 16)), rows_lds, s, out, in, (const T*)h->S[a], n, lines);
+            hipError_t e = done("dst_strip_rows_kernel");
+            return e == hipSuccess ? WHHD_OK : hip_fail(e, "dst strip rows kernel");
+        }
+        hipLaunchKernelGGL(dst_strip_kernel<T>, dim3((unsigned)((lines + 63) / 64), (all + 3) / 4), dim3(256), 0,
+                           s, out, in, (const T*)h->S[a], n, lines, m, si, sj, sb,
+                           scale ? (const T*)h->lam[0] : none, scale ? (const T*)h->lam[1] : none,
+                           scale ? (const T*)h->lam[2] : none, n2);
+        hipError_t e = done("dst_strip_kernel");
+        return e == hipSuccess ? WHHD_OK : hip_fail(e, "dst strip kernel");
     }
     dim3 grid((unsigned)((m + kTI - 1) / kTI), (unsigned)((n + kTK - 1) / kTK), nb);
     hipLaunchKernelGGL(dst_pass_kernel<T>, grid, dim3(256), 0, s, out, in, (const T*)h->S[a], n, m,
@@ -779,11 +951,23 @@ int dst3d_create_t(int n1, int n2, int n3, double dx, double dy, double dz, bool
                 S.push_back((T)-std::sin(2.0 * M_PI * k / M));
             }
         } else {
-            S.resize((size_t)n * n);
             const double sc = std::sqrt(2.0 / (n + 1));
-            for (int k = 0; k < n; ++k)
-                for (int j = 0; j < n; ++j)
-                    S[(size_t)k * n + j] = (T)(sc * std::sin(M_PI * (double)((int64_t)(k + 1) * (j + 1) % (2 * (n + 1))) / (n + 1)));
+            auto sine = [&](int k, int j) {
+                return sc * std::sin(M_PI * (double)((int64_t)(k + 1) * (j + 1) % (2 * (n + 1))) / (n + 1));
+            };
+            if (n <= kStripMax<T>) {
+                const int rows = (n + 1) / 2, even = strips<T>(rows) * kStrip<T>;
+                const int pitch = even + strips<T>(n / 2) * kStrip<T>;
+                S.assign((size_t)rows * pitch, T(0));
+                for (int k = 0; k < n; ++k)
+                    for (int j = 0; j < rows; ++j)
+                        S[(size_t)j * pitch + (k & 1 ? even : 0) + k / 2] =
+                            (T)(2 * j == n - 1 ? 0.5 * sine(k, j) : sine(k, j));
+            } else {
+                S.resize((size_t)n * n);
+                for (int k = 0; k < n; ++k)
+                    for (int j = 0; j < n; ++j) S[(size_t)k * n + j] = (T)sine(k, j);
+            }
         }
         for (int k = 0; k < n; ++k)
             lam[k] = (planar && a == 2) ? T(0)
@@ -842,11 +1026,14 @@ int dst3d_solve_t(const whhd_dst3d_s* h, T* phi, const T* b, hipStream_t s) {
     }
     TRY(dst_pass<T>(h, tmp, b, 0, s));
     TRY(dst_pass<T>(h, phi, tmp, 1, s));
-    TRY(dst_pass<T>(h, tmp, phi, 2, s));
-    hipLaunchKernelGGL(eigen_scale_kernel<T>, grid_xyz(h->n1, h->n2, h->n3), dim3(64, 4), 0, s, tmp,
-                       lam[0], lam[1], lam[2], h->n1, h->n2, h->n3);
-    hipError_t e = done("eigen_scale_kernel");
-    if (e != hipSuccess) return hip_fail(e, "eigen scale kernel");
+    const bool fused = !h->logm[2] && h->n3 <= kStripMax<T>;  // the strip kernel divides as it stores
+    TRY(dst_pass<T>(h, tmp, phi, 2, s, fused));
+    if (!fused) {
+        hipLaunchKernelGGL(eigen_scale_kernel<T>, grid_xyz(h->n1, h->n2, h->n3), dim3(64, 4), 0, s, tmp,
+                           lam[0], lam[1], lam[2], h->n1, h->n2, h->n3);
+        hipError_t e = done("eigen_scale_kernel");
+        if (e != hipSuccess) return hip_fail(e, "eigen scale kernel");
+    }
     TRY(dst_pass<T>(h, phi, tmp, 2, s));
     TRY(dst_pass<T>(h, tmp, phi, 1, s));
     return dst_pass<T>(h, phi, tmp, 0, s);
@@ -905,7 +1092,7 @@ int sweep3d_solve_t(whhd_sweep3d_t h, T* qx, T* qy, T* qz, const T* xv, const T*
     const bool d = h->bc == 'd';
     if (d && !zv) return fail(WHHD_INVALID_ARG, "sweep3d_solve: velocity bc 'd' needs zv");
     if (d)  // SetQxQyBoundary 'd': qy's bottom plane integrates zv along x
-        hipLaunchKernelGGL(bottom_qy_kernel<T>, dim3((h->ny + 255) / 256), dim3(256), 0, s, qy, zv,
+        hipLaunchKernelGGL(bottom_qy_kernel<T>, dim3((h->ny + 63) / 64), dim3(64), 0, s, qy, zv,
                            h->nx, h->ny, (T)h->dx);
     hipLaunchKernelGGL(sweep_kernel<T>, grid_xyz(h->nx + 1, h->ny + 1, 1), dim3(64, 4), 0, s, qx, qy,
                        qz, xv, yv, h->nx, h->ny, h->nz, (T)h->dz, d ? 1 : 0);
