@@ -59,6 +59,7 @@ struct Level {
     float *hx = nullptr, *hy = nullptr, *hz = nullptr;
     float* kf = nullptr;  // face spacing factors (face_factor_kernel)
     __half *axh = nullptr, *ayh = nullptr, *azh = nullptr;  // finest level: FP16 copies
+    float *inv = nullptr, *invh = nullptr;  // 1 / diagonal (0 where closed); invh with the FP16 copies
 };
 
 struct LevelArgs {
@@ -69,6 +70,7 @@ struct LevelArgs {
     // FP16 copies of the fractions (the finest level inside the tolerance
     // solve's V-cycles), or null
     const __half *axh, *ayh, *azh;
+    const float* inv;  // 1 / diagonal of the fractions the kernel reads
 };
 
 // Fraction j of a face array, from the FP16 copy when H16.
@@ -160,6 +162,45 @@ __global__ void jacobi_kernel(float* __restrict__ dst, const float* __restrict__
     stencil<Z, float, decltype(in), H16>(a, in, x, y, z, i, diag, off);
     const float v = in(i, 0, 0, 0);
     dst[i] = diag > 1e-12f ? (1.f - w) * v + w * (f[i] - off) / diag : 0.f;
+}
+
+// 1 / diagonal of every cell, 0 where all its faces are closed.
+template <bool Z, bool H16>
+__global__ void inv_diag_kernel(float* __restrict__ inv, LevelArgs a) {
+    const int y = blockIdx.x * 64 + threadIdx.x;
+    const int x = blockIdx.y * 4 + threadIdx.y;
+    const int z = blockIdx.z;
+    if (y >= a.ny || x >= a.nx) return;
+    const int64_t i = y + (int64_t)x * a.ny + (int64_t)z * a.nx * a.ny;
+    float diag, off;
+    auto none = [](int64_t, auto...) { return 0.f; };
+    stencil<Z, float, decltype(none), H16>(a, none, x, y, z, i, diag, off);
+    inv[i] = diag > 1e-12f ? 1.f / diag : 0.f;
+}
+
+// The first two sweeps from a zero iterate in one: the first leaves w f / diagonal
+// in every cell, which the second forms at the seven cells it reads from f and the
+// level's 1 / diagonal, so the first's pass over the fractions, its write and its
+// launch go.  Bound by its 14 + 7 loads per cell through L1 and the arrays' bytes
+// (192^3 with FP16 fractions: 31.7 + 27.5 us for the two sweeps, now 43.7; the three
+// levels below it 5 + 4.8 on average, now 6.2).  Forming both sweeps' halo in LDS and
+// taking the residual there too was tried: at 192^3 the wider tiles' repeated cells
+// cost more than the saved pass (a solve 5.4 ms against 4.5), on the small levels it
+// is the same time.
+template <bool Z, bool H16>
+__global__ void jacobi2_kernel(float* __restrict__ dst, const float* __restrict__ f, LevelArgs a, float w) {
+    const int y = blockIdx.x * 64 + threadIdx.x;
+    const int x = blockIdx.y * 4 + threadIdx.y;
+    const int z = blockIdx.z;
+    if (y >= a.ny || x >= a.nx) return;
+    const int64_t i = y + (int64_t)x * a.ny + (int64_t)z * a.nx * a.ny;
+    auto first = [&](int64_t j, auto...) {
+        const float q = a.inv[j], v = (w * f[j]) * q;
+        return q != 0.f ? v : 0.f;
+    };
+    float diag, off;
+    stencil<Z, float, decltype(first), H16>(a, first, x, y, z, i, diag, off);
+    dst[i] = diag > 1e-12f ? (1.f - w) * first(i) + w * (f[i] - off) / diag : 0.f;
 }
 
 // Coarsest-level sweeps in FP64 for at most 256 cells: one cell per thread,
@@ -940,7 +981,8 @@ LevelArgs args_of(const whhd_mgfrac3d_s* h, const Level& L) {
     const bool h16 = h->fp16_fine && L.axh;
     return LevelArgs{L.ax, L.ay, L.az, L.hx, L.hy, L.hz, L.d.x, L.d.y, L.d.z,
                      h->he[0], h->he[1], h->he[2], L.kf,
-                     h16 ? L.axh : nullptr, h16 ? L.ayh : nullptr, h16 ? L.azh : nullptr};
+                     h16 ? L.axh : nullptr, h16 ? L.ayh : nullptr, h16 ? L.azh : nullptr,
+                     h16 ? L.invh : L.inv};
 }
 
 hipError_t launch_status(const char* name) {
@@ -1015,7 +1057,24 @@ int smooth(const whhd_mgfrac3d_s* h, const Level& L, int n, float w, hipStream_t
     float* a = L.v;
     float* b = L.t;
     if (zero && n == 0) return fill(L.v, 0.f, cells(L.d), s);
-    for (int k = 0; k < n; ++k) {
+    int k = 0;
+    if (zero && n >= 2) {  // (never with C or a pair)
+        const LevelArgs la = args_of(h, L);
+        const dim3 g = grid_of(L.d.x, L.d.y, L.d.z), t(64, 4);
+        if (n & 1) std::swap(a, b);  // so that the last sweep ends in L.v
+        const bool h16 = la.axh != nullptr;
+        if (h->bc == 'z') {
+            if (h16) hipLaunchKernelGGL((jacobi2_kernel<true, true>), g, t, 0, s, a, L.f, la, w);
+            else hipLaunchKernelGGL((jacobi2_kernel<true, false>), g, t, 0, s, a, L.f, la, w);
+        } else {
+            if (h16) hipLaunchKernelGGL((jacobi2_kernel<false, true>), g, t, 0, s, a, L.f, la, w);
+            else hipLaunchKernelGGL((jacobi2_kernel<false, false>), g, t, 0, s, a, L.f, la, w);
+        }
+        hipError_t e = launch_status("mg_jacobi2_kernel");
+        if (e != hipSuccess) return hip_fail(e, "mg jacobi kernel");
+        k = 2;
+    }
+    for (; k < n; ++k) {
         if (C && k == 0) {
             TRY(jacobi(h, L, b, a, L.f, w, s, false, C));
             std::swap(a, b);
@@ -1249,6 +1308,29 @@ int mgfrac3d_create(const float* ax, const float* ay, const float* az, int nx, i
                            L.hz, L.d.x, L.d.y, L.d.z, h->he[0], h->he[1], h->he[2]);
         hipError_t e = launch_status("mg_face_factor_kernel");
         if (e != hipSuccess) st = hip_fail(e, "mgfrac3d_create: face factors");
+    }
+    for (size_t l = 0; l < h->lv.size() && st == WHHD_OK; ++l) {
+        Level& L = h->lv[l];
+        const dim3 g = grid_of(L.d.x, L.d.y, L.d.z), t(64, 4);
+        const size_t bytes = (size_t)cells(L.d) * 4;
+        L.inv = (float*)alloc(bytes);
+        if (l == 0) L.invh = (float*)alloc(bytes);
+        if (!L.inv || (l == 0 && !L.invh)) {
+            st = fail(WHHD_OOM, "mgfrac3d_create: allocation failed");
+            break;
+        }
+        h->fp16_fine = false;
+        if (h->bc == 'z') hipLaunchKernelGGL((inv_diag_kernel<true, false>), g, t, 0, s, L.inv, args_of(h, L));
+        else hipLaunchKernelGGL((inv_diag_kernel<false, false>), g, t, 0, s, L.inv, args_of(h, L));
+        if (l == 0) {
+            h->fp16_fine = true;
+            const LevelArgs ah = args_of(h, L);
+            h->fp16_fine = false;
+            if (h->bc == 'z') hipLaunchKernelGGL((inv_diag_kernel<true, true>), g, t, 0, s, L.invh, ah);
+            else hipLaunchKernelGGL((inv_diag_kernel<false, true>), g, t, 0, s, L.invh, ah);
+        }
+        hipError_t e = launch_status("mg_inv_diag_kernel");
+        if (e != hipSuccess) st = hip_fail(e, "mgfrac3d_create: diagonals");
     }
     if (st == WHHD_OK) {
         const dim3 g = grid_of(nx, ny, nz);
