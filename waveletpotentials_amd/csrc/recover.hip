@@ -100,9 +100,10 @@ __global__ void cut_kernel(float* qx, float* qy, float* qz, int nx, int ny, int 
 // separable transforms commute, so the order changes only FP32 rounding; the
 // orders are the fastest of those measured at 256^3 (forward y, x, z against
 // x, y, z: 0.697 vs 0.705 ms; inverse z, y, x against x, y, z: 0.695 vs
-// 0.698 ms).  The line-parallel kernels read and write different arrays, so
-// the passes of the standard order ping-pong: in -> out -> scratch -> out.
-// `scratch` may be `in` (consumed by the first pass) but not `out`.
+// 0.698 ms, each array by itself).  Line-parallel passes of the standard order
+// read and write different arrays and ping-pong: in -> out -> scratch -> out;
+// `scratch` may be `in` (consumed by the first pass) but not `out`.  Passes in
+// interleaved order need no second array (in_place_passes).
 struct Pass {
     char bc;
     int wt;

@@ -416,10 +416,14 @@ int eikonal_sweep(float* ls, float* scratch, int nx, int ny, int nz, double h, i
     // relaxations, a stream being captured, no memory) every tile runs
     uint8_t* flags = nullptr;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (n_iters >= 8 && hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
-        hipMallocAsync((void**)&flags, 2 * tiles, s) != hipSuccess) {
-        (void)hipGetLastError();
-        flags = nullptr;
+    if (n_iters >= 8) {
+        const hipError_t e = hipStreamIsCapturing(s, &cap);
+        if (e == hipSuccess && cap == hipStreamCaptureStatusNone &&
+            hipMallocAsync((void**)&flags, 2 * tiles, s) != hipSuccess) {
+            (void)hipGetLastError();
+            flags = nullptr;
+        }
+        if (e != hipSuccess) (void)hipGetLastError();
     }
     const bool wide = (int64_t)nx * ny * nz * 4 >= (int64_t)1 << 31;
     for (int i = 0; i < n_iters; ++i) {
