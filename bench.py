@@ -9,7 +9,9 @@ Prints one JSON line.  `value` is Mcells/s of the whole solve (K solves
 between device synchronizations).  `roofline` describes the kernel with the
 largest share of the solve: a second run of K solves records HIP events after
 every launch on the stream the library launches on (the library's stage
-trace), giving each launch's duration in context.  `cpu_baseline` times the
+trace; it then launches every array's pass by itself, where a timed solve
+takes the three components of a pass together), giving each launch's duration
+in context.  `cpu_baseline` times the
 C oracle (a port of the reference algorithm) built in FP32 on this host, with
 the FP64 oracle's figure beside it.  The line also carries `learned_init`
 (the learned initial guess against the multigrid from zero on held-out 192^3
@@ -21,6 +23,7 @@ with a V-cycle preconditioner; `--workload` runs any of them alone).
 import argparse
 import json
 import os
+import re
 import sys
 import time
 
@@ -74,14 +77,22 @@ def stage_bytes(stage, ab):
 def measured_traffic(kernel):
     """HBM bytes per launch of `kernel` from the committed rocprof counter
     summary (FETCH_SIZE and WRITE_SIZE runs, each scaled by the calibration
-    kernel's reading), or None when the summary does not cover it."""
+    kernel's reading), or None when the summary does not cover it.  The summary
+    lists a line-parallel kernel with both wavelets of its pair and names the
+    strided kernel that writes the interleaved order apart."""
     path = os.path.join(ROOT, "profiles", "traffic_recover3d_256.json")
     try:
         with open(path) as f:
             rows = json.load(f)
     except (OSError, ValueError):
         return None
-    row = rows.get("kernels", {}).get(kernel)
+    kernels = rows.get("kernels", {})
+    row = kernels.get(kernel)
+    m = re.match(r"lp_kernel<([^,]+),(.*)>$", kernel)
+    for name, r in kernels.items() if m and not row else ():
+        k = re.match(r"lp_kernel<([^,]+),(.*)>$", name)
+        if k and m.group(1) in k.group(1).split(" + ") and k.group(2).replace("interleaved", "strided") == m.group(2):
+            row = r
     if not row:
         return None
     return {"bytes": int(row["fetch_bytes"] + row["write_bytes"]),
@@ -182,7 +193,7 @@ def main():
         "dtype": "f32",
         "data": "synthetic (curl of a seeded Fourier potential, |k|<=16, |k|^-11/6)",
         "config": {"workload": f"3D vector-potential recovery {N}^3 MAC grid, curl CDF3.7 'n', "
-                               f"div CDF4.6 'd', {len(stages)} launches", "cells": cells},
+                               f"div CDF4.6 'd', {len(stages)} passes", "cells": cells},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic["bytes"] if traffic else None,

@@ -120,7 +120,9 @@ typedef struct whhd_recover3d_s* whhd_recover3d_t;
 /* CuWaveletPotentialRecover3D(int3 dim, DTYPE3 dx, char bc, WaveletType curl,
  * WaveletType div) (WaveletPotentials/cuWaveletPotentialRecover3D.cuh:12,
  * .cu:6-12).  Allocates the handle's scratch: one velocity-sized and one
- * potential-sized array per component (passes run out of place). */
+ * potential-sized array per component (a solve works in place in the velocity-sized
+ * ones where the line-parallel kernels cover its lengths and wavelets, out of place
+ * otherwise). */
 WHHD_API int whhd_recover3d_create(int nx, int ny, int nz, double dx, double dy, double dz,
                                    char bc, int wavelet_curl, int wavelet_div,
                                    whhd_recover3d_t* out);

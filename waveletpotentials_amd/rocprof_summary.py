@@ -27,24 +27,27 @@ CAL_BYTES = 16 * 1024 * 1024 * 4  # calibration kernel: bytes read and bytes wri
 CAL_NAME = "vectorized_elementwise_kernel"
 CAL_OP = "MulFunctor<float>"  # torch.mul(src, 1.0, out=dst) on FP32 tensors
 
-_WT = {"Cdf37": "cdf3.7 n", "Cdf46": "cdf4.6 d"}
+_WT = {("HalfN", "37"): "cdf3.7 n", ("HalfD", "37"): "cdf3.7 d", ("HalfN", "35"): "cdf3.5 n",
+       ("HalfD", "35"): "cdf3.5 d", ("WholeN", "46"): "cdf4.6 n", ("WholeD44", "46"): "cdf4.6 d",
+       ("WholeN", "44"): "cdf4.4 n", ("WholeD44", "44"): "cdf4.4 d"}
+_WT_TILE = {"Cdf37": "cdf3.7 n", "Cdf46": "cdf4.6 d"}
 
 
 def kernel_label(name):
-    """The label the library's stage trace uses for a kernel symbol."""
-    m = re.search(r"lp_kernel.*Up(Cdf\d\d)E.*ELi(\d)ELi(\d)ELb([01])ELb([01])E", name)
+    """The label the library's stage trace uses for a kernel symbol.  One line-parallel
+    kernel holds both wavelets of a pair: its label lists them (`a + b`)."""
+    m = (re.search(r"lp_kernel.*?\d+Ix(\w+?)ENS_\d+UpCdf(\d\d)E.*\d+Ix(\w+?)ENS_\d+UpCdf(\d\d)E"
+                   r".*ELi(\d)ELb([01])ELi(\d)E", name)
+         or re.search(r"lp_kernel<.*?Ix(\w+), .*?UpCdf(\d\d),.*Ix(\w+), .*?UpCdf(\d\d),.*>, (\d), (true|false), (\d)>",
+                      name))
     if m:
-        return (f"lp_kernel<{_WT.get(m.group(1), m.group(1))},L={m.group(2)},"
-                f"{'fwd' if m.group(4) == '1' else 'inv'},"
-                f"{'contiguous' if m.group(5) == '1' else 'strided'}>")
-    m = re.search(r"lp_kernel<.*Up(Cdf\d\d),.*>, (\d), (\d), (true|false), (true|false)>", name)
-    if m:
-        return (f"lp_kernel<{_WT.get(m.group(1), m.group(1))},L={m.group(2)},"
-                f"{'fwd' if m.group(4) == 'true' else 'inv'},"
-                f"{'contiguous' if m.group(5) == 'true' else 'strided'}>")
+        a, b = ((m.group(k), m.group(k + 1)) for k in (1, 3))
+        return (f"lp_kernel<{_WT.get(a, '/'.join(a))} + {_WT.get(b, '/'.join(b))},L={m.group(5)},"
+                f"{'fwd' if m.group(6) in ('1', 'true') else 'inv'},"
+                f"{('contiguous', 'strided', 'interleaved')[int(m.group(7))]}>")
     m = re.search(r"line_tile_kernel.*Up(Cdf\d\d)E.*EE([fd])Lb([01])ELb([01])E", name)
     if m:
-        return (f"line_tile_kernel<{_WT.get(m.group(1), m.group(1))},"
+        return (f"line_tile_kernel<{_WT_TILE.get(m.group(1), m.group(1))},"
                 f"{'f32' if m.group(2) == 'f' else 'f64'},{'fwd' if m.group(3) == '1' else 'inv'},"
                 f"{'strided' if m.group(4) == '1' else 'contiguous'}>")
     m = re.search(r"unet\d+(conv3_wgrad_kernel|conv3_kernel)I((?:L[ib]\d+E)+)E", name)
