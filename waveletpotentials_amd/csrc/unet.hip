@@ -639,8 +639,11 @@ __global__ void down_kernel(float* __restrict__ out, const float* __restrict__ i
 // A (64, 4) block over (y, x) and four z planes (the extents are multiples of 4):
 // the FP64 scale, whose square root had cost more than the rest of a cell, is
 // formed once per workgroup, the x and y weights once per column (192^3 from
-// 48^3: 35 -> 19 us).
+// 48^3: 35 -> 19 us).  P2: F is a power of two, so 1 / F is exact and the coordinate a
+// product; else it is divided (192^3 by 4 that way 21 us), since the reciprocal's
+// rounding would move it and cells on coarse centres would mix two values.
 constexpr int kUpZ = 4;
+template <bool P2>
 __global__ void __launch_bounds__(256) up_kernel(float* __restrict__ p, const float* __restrict__ out,
                                                  const double* __restrict__ stats, float len2, int Zc,
                                                  int Xc, int Yc, int F) {
@@ -651,7 +654,8 @@ __global__ void __launch_bounds__(256) up_kernel(float* __restrict__ p, const fl
     const int y = blockIdx.x * 64 + threadIdx.x, x = blockIdx.y * 4 + threadIdx.y;
     const float inv_f = 1.f / (float)F;
     auto axis = [&](int c, int nc, int& c0, int& c1, float& w) {
-        float u = ((float)c + 0.5f) * inv_f - 0.5f;
+        const float v = (float)c + 0.5f;
+        float u = (P2 ? v * inv_f : v / (float)F) - 0.5f;
         u = fminf(fmaxf(u, 0.f), (float)(nc - 1));
         c0 = (int)u;
         c1 = c0 + 1 < nc ? c0 + 1 : c0;
@@ -1157,7 +1161,7 @@ WHHD_API int whhd_unet_predict(whhd_unet_t h, float* p0, const float* f, const f
         hipLaunchKernelGGL(unet::output_kernel, unet::g1(h->V[0]), dim3(256), 0, st, p0, h->out,
                            unet::stats(h), len2, h->V[0]);
     else
-        hipLaunchKernelGGL(unet::up_kernel,
+        hipLaunchKernelGGL((h->factor & (h->factor - 1) ? unet::up_kernel<false> : unet::up_kernel<true>),
                            dim3((h->ny * h->factor + 63) / 64, (h->nx * h->factor + 3) / 4,
                                 h->nz * h->factor / unet::kUpZ),
                            dim3(64, 4), 0, st, p0, h->out, unet::stats(h), len2, h->nz, h->nx, h->ny,
