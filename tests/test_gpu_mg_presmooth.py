@@ -48,3 +48,25 @@ def test_pcg_reaches_tolerance(whhd, orc, n, bc, nu):
     v = hi.double().cpu().numpy() + lo.double().cpu().numpy()
     r_ref = orc.mg_rel_residual(v, f.astype(np.float32).astype(np.float64), *fr, h, bc)
     assert r_ref <= 1e-6 * (1 + 1e-3) + 1e-7
+
+
+def test_create_allocates_what_a_solve_reads(whhd):
+    """The device memory of a 192^3 handle: per level three cell arrays, the faces, and
+    the reciprocal diagonals of the levels that are launched one by one (the finest in
+    its FP16 form only); on the finest level FP16 faces and three more cell arrays.
+    12 MB on top for the allocations' granularity and the small tables; one unread
+    cell array of the finest level is 28 MB."""
+    n = 192
+    fr = [torch.ones(s, device="cuda") for s in ((n, n + 1, n), (n, n, n + 1), (n + 1, n, n))]
+    h = (1.0 / n,) * 3
+    del_first = whhd.CuMultigridFrac3D(*fr, (n, n, n), h, "n")   # the runtime's own first-use memory
+    del del_first
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    mg = whhd.CuMultigridFrac3D(*fr, (n, n, n), h, "n")
+    used = before - torch.cuda.mem_get_info()[0]
+    want = 0
+    for l, (x, y, z) in enumerate(mg.levels()):
+        cells, faces = x * y * z, (x + 1) * y * z + x * (y + 1) * z + x * y * (z + 1)
+        want += 4 * (3 * cells + faces) + (4 * 4 * cells + 2 * faces if l == 0 else 4 * cells)
+    assert used <= want + (12 << 20), (used, want)

@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <vector>
 
 #include "whhd_internal.h"
@@ -59,7 +60,10 @@ struct Level {
     float *hx = nullptr, *hy = nullptr, *hz = nullptr;
     float* kf = nullptr;  // face spacing factors (face_factor_kernel)
     __half *axh = nullptr, *ayh = nullptr, *azh = nullptr;  // finest level: FP16 copies
-    float *inv = nullptr, *invh = nullptr;  // 1 / diagonal (0 where closed); invh with the FP16 copies
+    // 1 / diagonal (0 where closed) of the fractions that sweeps from a zero iterate
+    // read, the FP16 copies on the finest level; not filled where no kernel reads it:
+    // the coarsest level and those inside the one-workgroup cycle
+    float* inv = nullptr;
 };
 
 struct LevelArgs {
@@ -70,7 +74,7 @@ struct LevelArgs {
     // FP16 copies of the fractions (the finest level inside the tolerance
     // solve's V-cycles), or null
     const __half *axh, *ayh, *azh;
-    const float* inv;  // 1 / diagonal of the fractions the kernel reads
+    const float* inv;  // 1 / diagonal of the fractions the kernel reads, or null
 };
 
 // Fraction j of a face array, from the FP16 copy when H16.
@@ -982,7 +986,7 @@ LevelArgs args_of(const whhd_mgfrac3d_s* h, const Level& L) {
     return LevelArgs{L.ax, L.ay, L.az, L.hx, L.hy, L.hz, L.d.x, L.d.y, L.d.z,
                      h->he[0], h->he[1], h->he[2], L.kf,
                      h16 ? L.axh : nullptr, h16 ? L.ayh : nullptr, h16 ? L.azh : nullptr,
-                     h16 ? L.invh : L.inv};
+                     h16 == (L.axh != nullptr) ? L.inv : nullptr};
 }
 
 hipError_t launch_status(const char* name) {
@@ -1058,8 +1062,8 @@ int smooth(const whhd_mgfrac3d_s* h, const Level& L, int n, float w, hipStream_t
     float* b = L.t;
     if (zero && n == 0) return fill(L.v, 0.f, cells(L.d), s);
     int k = 0;
-    if (zero && n >= 2) {  // (never with C or a pair)
-        const LevelArgs la = args_of(h, L);
+    const LevelArgs la = args_of(h, L);
+    if (zero && n >= 2 && la.inv) {  // (never with C or a pair)
         const dim3 g = grid_of(L.d.x, L.d.y, L.d.z), t(64, 4);
         if (n & 1) std::swap(a, b);  // so that the last sweep ends in L.v
         const bool h16 = la.axh != nullptr;
@@ -1081,7 +1085,6 @@ int smooth(const whhd_mgfrac3d_s* h, const Level& L, int n, float w, hipStream_t
             continue;
         }
         if (hi && k == n - 1) {
-            const LevelArgs la = args_of(h, L);
             const dim3 pg = grid_of(L.d.x, L.d.y, L.d.z), pb(64, 4);
             const bool h16 = la.axh != nullptr;
             if (h->bc == 'z') {
@@ -1217,6 +1220,16 @@ int mgfrac3d_create(const float* ax, const float* ay, const float* az, int nx, i
         h->owned.push_back(p);
         return p;
     };
+    // k arrays of n floats in one allocation, each 256-byte aligned: a large hipMalloc
+    // and its hipFree take about 300 us, and every solid that moves pays for a handle
+    auto alloc_cells = [&](size_t n, std::initializer_list<float**> to) {
+        const size_t pitch = (n + 63) & ~(size_t)63;
+        float* p = (float*)alloc(pitch * to.size() * 4);
+        for (float** q : to) {
+            *q = p;
+            if (p) p += pitch;
+        }
+    };
     hipStream_t s = nullptr;
     Dim3 d = {nx, ny, nz}, last = d;
     int min_dim = std::min(nx, std::min(ny, nz));
@@ -1225,9 +1238,7 @@ int mgfrac3d_create(const float* ax, const float* ay, const float* az, int nx, i
         Level L;
         L.d = d;
         const size_t n = (size_t)cells(d);
-        L.f = (float*)alloc(n * 4);
-        L.v = (float*)alloc(n * 4);
-        L.t = (float*)alloc(n * 4);
+        alloc_cells(n, {&L.f, &L.v, &L.t, &L.inv});
         L.ax = (float*)alloc((size_t)(d.x + 1) * d.y * d.z * 4);
         L.ay = (float*)alloc((size_t)d.x * (d.y + 1) * d.z * 4);
         L.az = (float*)alloc((size_t)d.x * d.y * (d.z + 1) * 4);
@@ -1309,42 +1320,16 @@ int mgfrac3d_create(const float* ax, const float* ay, const float* az, int nx, i
         hipError_t e = launch_status("mg_face_factor_kernel");
         if (e != hipSuccess) st = hip_fail(e, "mgfrac3d_create: face factors");
     }
-    for (size_t l = 0; l < h->lv.size() && st == WHHD_OK; ++l) {
-        Level& L = h->lv[l];
-        const dim3 g = grid_of(L.d.x, L.d.y, L.d.z), t(64, 4);
-        const size_t bytes = (size_t)cells(L.d) * 4;
-        L.inv = (float*)alloc(bytes);
-        if (l == 0) L.invh = (float*)alloc(bytes);
-        if (!L.inv || (l == 0 && !L.invh)) {
-            st = fail(WHHD_OOM, "mgfrac3d_create: allocation failed");
-            break;
-        }
-        h->fp16_fine = false;
-        if (h->bc == 'z') hipLaunchKernelGGL((inv_diag_kernel<true, false>), g, t, 0, s, L.inv, args_of(h, L));
-        else hipLaunchKernelGGL((inv_diag_kernel<false, false>), g, t, 0, s, L.inv, args_of(h, L));
-        if (l == 0) {
-            h->fp16_fine = true;
-            const LevelArgs ah = args_of(h, L);
-            h->fp16_fine = false;
-            if (h->bc == 'z') hipLaunchKernelGGL((inv_diag_kernel<true, true>), g, t, 0, s, L.invh, ah);
-            else hipLaunchKernelGGL((inv_diag_kernel<false, true>), g, t, 0, s, L.invh, ah);
-        }
-        hipError_t e = launch_status("mg_inv_diag_kernel");
-        if (e != hipSuccess) st = hip_fail(e, "mgfrac3d_create: diagonals");
-    }
     if (st == WHHD_OK) {
         const dim3 g = grid_of(nx, ny, nz);
         h->rblocks = (int64_t)g.x * g.y * g.z;
-        h->r = (float*)alloc((size_t)cells(h->dim) * 4);
+        alloc_cells((size_t)cells(h->dim), {&h->r, &h->pcg_p[0], &h->pcg_p[1]});
         h->part = (double*)alloc((2 * kNormBlocks + 2) * sizeof(double));
         h->cbuf = (double*)alloc((size_t)cells(h->lv.back().d) * 2 * sizeof(double));
         h->rpart = (double*)alloc((size_t)(2 * h->rblocks + 2) * sizeof(double));
         h->fac64 = (double*)alloc((size_t)2 * (nx + ny + nz) * sizeof(double));
-        h->pcg_p[0] = (float*)alloc((size_t)cells(h->dim) * 4);
-        h->pcg_p[1] = (float*)alloc((size_t)cells(h->dim) * 4);
         h->coef = (double*)alloc(4 * sizeof(double));
-        if (!h->r || !h->part || !h->cbuf || !h->rpart || !h->fac64 || !h->pcg_p[0] || !h->pcg_p[1] ||
-            !h->coef)
+        if (!h->r || !h->part || !h->cbuf || !h->rpart || !h->fac64 || !h->coef)
             st = fail(WHHD_OOM, "mgfrac3d_create: allocation failed");
     }
     if (st == WHHD_OK) {
@@ -1394,6 +1379,24 @@ int mgfrac3d_create(const float* ax, const float* ay, const float* az, int nx, i
             h->small_lds = (size_t)off * sizeof(float);
             if (st == WHHD_OK && h->small_lds <= 60 * 1024) h->fuse_from = from;
         }
+    }
+    const size_t smoothed = h->fuse_from >= 0 ? (size_t)h->fuse_from : h->lv.size() - 1;
+    for (size_t l = 0; l < smoothed && st == WHHD_OK; ++l) {
+        Level& L = h->lv[l];
+        const dim3 g = grid_of(L.d.x, L.d.y, L.d.z), t(64, 4);
+        h->fp16_fine = true;
+        const LevelArgs a = args_of(h, L);
+        h->fp16_fine = false;
+        const bool h16 = a.axh != nullptr;
+        if (h->bc == 'z') {
+            if (h16) hipLaunchKernelGGL((inv_diag_kernel<true, true>), g, t, 0, s, L.inv, a);
+            else hipLaunchKernelGGL((inv_diag_kernel<true, false>), g, t, 0, s, L.inv, a);
+        } else {
+            if (h16) hipLaunchKernelGGL((inv_diag_kernel<false, true>), g, t, 0, s, L.inv, a);
+            else hipLaunchKernelGGL((inv_diag_kernel<false, false>), g, t, 0, s, L.inv, a);
+        }
+        hipError_t e = launch_status("mg_inv_diag_kernel");
+        if (e != hipSuccess) st = hip_fail(e, "mgfrac3d_create: diagonals");
     }
     if (st == WHHD_OK) {
         // uniform finest spacing: interior faces 2 / (2 h h), wall faces 2 / ((e + h) h)
