@@ -439,18 +439,22 @@ struct Wavelet {
 };
 
 // y = M x over lanes 0..M-1 (lane r gets row r); other lanes return row 0.
-// Each lane loads its own row: M loads in flight together, the same for every
-// line a wavefront lifts (selecting the row from scalar loads of the whole
-// matrix waited for four of them in turn).
+// The row is selected from scalar loads of the whole matrix.  A row loaded by each
+// lane instead is faster for a few lines (2D recovery of 128^2 23.8 against 24.2 us)
+// but slower for many short ones (16384 strided lines of 4 samples 5.3 against 4.5 us)
+// and for long strided ones (4096 samples 26 against 24).
 template <int M, const double* Mat, class T>
 WHHD_DEV T apply_l10(T v, int lane) {
-    const double* row = Mat + (lane < M ? lane : 0) * M;
-    T coef[M];
-#pragma unroll
-    for (int c = 0; c < M; ++c) coef[c] = T(row[c]);
+    const int r = lane < M ? lane : 0;
     T acc = T(0);
 #pragma unroll
-    for (int c = 0; c < M; ++c) acc += lane_get(v, c) * coef[c];
+    for (int c = 0; c < M; ++c) {
+        T xc = lane_get(v, c);
+        T coef = T(0);
+#pragma unroll
+        for (int rr = 0; rr < M; ++rr) coef = (r == rr) ? T(Mat[rr * M + c]) : coef;
+        acc += xc * coef;
+    }
     return acc;
 }
 
