@@ -6,7 +6,9 @@ together.
 Transforms: against the windowed kernels (the general path) on unconstrained
 input, so that samples the boundary reflections ignore are covered too, and
 against the FP64 oracle on admissible input.  Line counts of 64 k + r put
-partial wavefronts at the end of the array.  Tolerances: FP32 roundoff over at
+partial wavefronts at the end of the array.  A single array of few lines of 2^6
+samples or more runs the windowed kernels by itself: the second test has the counts
+from which such lines run the line-parallel ones, and the counts below.  Tolerances: FP32 roundoff over at
 most eight lifting levels, 2e-6 relative to the FP64 oracle, hence twice that
 between two FP32 paths.  Recovery: 1e-5 to the oracle, the path's stated bar.
 """
@@ -71,12 +73,45 @@ def test_line_parallel_equals_windowed(whhd, orc, wt, bc, axis):
             assert rel([got[0]], [ref]) < TOL32, (n, m1, m2)
 
 
+@pytest.mark.parametrize("wt", ["cdf3.7", "cdf4.6", "cdf3.5", "cdf4.4"])
+@pytest.mark.parametrize("bc", ["n", "d"])
+@pytest.mark.parametrize("axis", ["y", "x", "z"])
+def test_few_and_many_long_lines(whhd, wt, bc, axis):
+    """Lines of 2^6..2^8 samples: up to 2048 of them (4096 contiguous ones, and x lines
+    with fewer than 16 neighbours in memory) one line per wavefront, the windowed
+    kernels' bits; more of them a line per lane, the same to FP32 rounding."""
+    rng = np.random.default_rng(23)
+    fw = whhd.CuWHHDForward.GetInstance()
+    L = whhd.lib()
+    for levels in (6, 7, 8):
+        n = line_len(wt, levels)
+        for m1, m2 in ((1, 1), (64, 32), (1, 2048), (683, 3), (65, 63), (8, 512), (8, 513), (241, 17)):
+            shape = {"y": (m2, m1, n), "x": (m2, n, m1), "z": (n, m1, m2)}[axis]
+            few = m1 * m2 <= (4096 if axis == "y" or (axis == "x" and m1 < 16) else 2048)
+            nz, nx, ny = shape
+            x = cuda(rng.standard_normal(shape))
+            for fwd in (True, False):
+                got = []
+                for mode in (0, 1):
+                    assert L.whhd_set_line_kernel(mode) == 0
+                    try:
+                        dst = torch.full(shape, float("nan"), device="cuda")
+                        fw.Solve1D(dst, x, (nx, ny, nz), levels, axis, bc, wtype(whhd, wt), fwd)
+                        torch.cuda.synchronize()
+                    finally:
+                        L.whhd_set_line_kernel(0)
+                    got.append(dst.cpu().numpy())
+                assert rel([got[0]], [got[1]]) < 2 * TOL32, (n, m1, m2, fwd)
+                if few:
+                    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)), (n, m1, m2, fwd)
+
+
 @pytest.mark.parametrize("pair", PAIRS, ids=["37-46", "35-44"])
 @pytest.mark.parametrize("bc", ["n", "d"])
 @pytest.mark.parametrize("n", [(8, 8, 8), (16, 8, 32), (4, 16, 8), (32, 64, 8), (64, 64, 64)])
 def test_recover3d_pairs_match_oracle(whhd, orc, pair, bc, n):
-    """Both forms of Solve; (4, 16, 8) has an axis below the line-parallel
-    kernels' range, so that axis runs the windowed ones."""
+    """Both forms of Solve; (4, 16, 8) has an x axis below the line-parallel kernels'
+    range, so that grid is solved out of place, array by array."""
     nx, ny, nz = n
     dx = tuple(1.0 / v for v in n)
     rng = np.random.default_rng(nx + ny)

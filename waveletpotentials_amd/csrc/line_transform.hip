@@ -247,11 +247,34 @@ static hipError_t launch_w(T* dst, const T* src, const LineGeom& g, bool fwd, bo
 
 // Arrays of up to 4096 lines get four lines (one per wavefront) a workgroup:
 // with the larger tiles, which suit the memory system, they occupy a few CUs
-// and every wavefront lifts several lines one after the other.
+// and every wavefront lifts several lines one after the other (4096 strided FP32
+// lines of 128 samples, 16 a tile, 22 us, 4 a tile 8).  Strided tiles that are no
+// wider than eight already keep every wavefront to two lines, and lose more in
+// their 16-byte rows from about 3500 lines on (FP64, 256 samples: 3072 lines 13.0 us
+// by eight, 12.0 by four; 4096 lines 13.6 and 15.0).
 static void few_lines(TileConfig& c, int64_t lines) {
-    if (lines > 4096) return;
-    if (c.strided_tile > 4) c.strided_tile = 4;
-    if (c.contig_tile > 4) c.contig_tile = 4;
+    if (lines <= (c.strided_tile > 8 ? 4096 : 3072) && c.strided_tile > 4) c.strided_tile = 4;
+    if (lines <= 4096 && c.contig_tile > 4) c.contig_tile = 4;
+}
+
+// Whether an array's lines are transformed faster a line per lane.  A lane walks its
+// line alone, 12-13 us for 256 samples however few the lines are; one line per
+// wavefront is done sooner while the lines are few and have 64 samples or more.  us,
+// line per lane / windowed, strided lines: 256 samples, 64 lines 12.4 / 6.0, 2048 lines
+// 12.9 / 9, 4096 13.2 / 14; 128: 7.2 / 4.7, 7.5 / 6.5, 7.6 / 8.5; 64: 4.6 / 4.0, 4.8 / 4.6,
+// 4.9 / 5.6; 32: 3.3 / 3.5, 3.5 / 3.8.  Contiguous lines, 4096 of 256, 128, 64 samples: 13.2 /
+// 7.5, 7.6 / 5.8, 5.0 / 4.7; 16 of 33 samples, inverse: 5.0 / 3.9, 256 of them 4.0 / 3.8.  x lines of arrays that are narrow along y have few
+// neighbours in memory, and a load of 64 lanes touches up to 64 cache lines (ny = 1, 2,
+// 4, 8: 4096 lines of 256 samples 56, 42, 17, 15 us a line per lane, windowed 18, 13, 11,
+// 11; 256 lines of 32 samples, ny = 1: 9.5 and 3.5).
+static bool lines_per_lane(int levels, char axis, int ny, int64_t lines) {
+    switch (axis) {
+    case 'y': case 'Y': return levels < 5 || lines > (levels == 5 ? 256 : 4096);
+    case 'x': case 'X':
+        if (ny < 16) return lines > 4096;
+        break;
+    }
+    return levels < 6 || lines > 2048;
 }
 
 template <class T>
@@ -300,7 +323,8 @@ int transform_lines(T* dst, const T* src, int nx, int ny, int nz, int levels, ch
     st = check_line(n, levels, wt);
     if (st != WHHD_OK) return st;
     if constexpr (sizeof(T) == sizeof(float)) {
-        if ((!cfg || cfg->allow_line_parallel) && g_line_kernel_mode.load() == 0) {
+        if ((!cfg || cfg->allow_line_parallel) && g_line_kernel_mode.load() == 0 &&
+            lines_per_lane(levels, axis, ny, (int64_t)nx * ny * nz / n * b.nb)) {
             const LineJob job{(float*)dst, (const float*)src, nx, ny, nz, bc, wt, b.stride};
             const int r = lp_transform(&job, 1, levels, axis, fwd, false, stream, b.waves, b.nb);
             if (r != -1) return r;
