@@ -1,8 +1,10 @@
-"""The DST solver's kernels at the lengths where they change: a line per lane (FP32,
-3..255 samples of 2^k - 1, partial wavefronts, contiguous lines from buffers that
-are and are not 16-byte aligned), the folded sine products (even and odd lengths
-around the strip widths and the largest folded length, with and without the staged
-rows) and the tiled product beyond them.
+"""The DST solver's kernels at the lengths and line counts where they change: a line
+per lane (FP32, 3..127 samples of 2^k - 1, and 255 from 8192 lines or 12288 contiguous
+ones up; partial wavefronts, contiguous lines from buffers that are and are not
+16-byte aligned), the half-wavefront transform below those counts, the folded sine
+products (even and odd lengths around the strip widths and the largest folded length;
+contiguous lines from memory up to 2^20 samples, staged in LDS above them) and the
+tiled product beyond them (also for contiguous lines where neither pays).
 
 Against dense FP64 sine transforms.  Tolerances: FP32 2e-5 relative, a few units
 of roundoff per pass times the spread of the eigenvalues' reciprocals; FP64 1e-12.
@@ -14,7 +16,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(3, 3, 3), (7, 15, 1), (255, 5, 31), (63, 127, 9), (15, 255, 65), (31, 7, 127), (2, 5, 6),
-          (16, 17, 33), (32, 31, 30), (97, 8, 64), (130, 129, 66), (4, 320, 5), (3, 321, 2), (257, 3, 5)]
+          (16, 17, 33), (32, 31, 30), (97, 8, 64), (130, 129, 66), (4, 320, 5), (3, 321, 2), (257, 3, 5),
+          (255, 91, 91), (111, 255, 111), (97, 85, 255),      # 255 samples, a line per lane
+          (115, 96, 110), (81, 200, 160), (70, 201, 70), (40, 318, 101)]  # contiguous: LDS rows, tiled
 
 
 def solve_dense(b, h):

@@ -231,11 +231,17 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
 }  // namespace dstl
 
 // One DST-I pass of `lines` lines of 2^logm - 1 samples, as dst_fft_kernel's
-// arguments describe them; false where no kernel applies.
+// arguments describe them; false where no kernel applies, or where dst_fft_kernel's
+// half-wavefront per line is faster: a lane's 255 samples take 13 us however few the
+// lines are (us a pass, line per lane against it: strided, up to 4098 lines +4, 8194
+// -1.5, 16386 -10; contiguous, up to 4098 lines +6, 8194 +2, 16386 -7; a planar 255^2
+// solve 65 against 41).  Shorter lines are faster a line per lane at every count
+// (127 samples 16 lines -3, 63 samples -7, contiguous -6 and -13).
 bool dst_lines(int logm, bool contig, float* out, const float* in, int64_t lines, int64_t n_inner,
                int64_t s_inner, int64_t s_outer, int64_t step, float c, const float* lam_q,
                const float* lam_r, const float* lam_s, int64_t lam_div, int reps, hipStream_t s) {
     const int64_t n = (1 << logm) - 1;
+    if (logm == 8 && lines < (contig ? 12288 : 8192)) return false;
     if (logm < 2 || logm > 8 || lines < 1 || lines * n >= (int64_t)1 << 31) return false;
     if (contig && (((uintptr_t)in | (uintptr_t)out) & 15)) return false;  // 16-byte copies
     const dstl::Args a{out, in, (uint32_t)lines, (uint32_t)n_inner, (uint32_t)s_inner, (uint32_t)s_outer,

@@ -862,8 +862,8 @@ int dst_pass(const whhd_dst3d_s* h, T* out, const T* in, int a, hipStream_t s,
         }
         const T c = (T)std::sqrt(2.0 / M);
         if constexpr (!is64<T>()) {
-            // 255^3 462 -> 213 us a solve, 127^3 96 -> 60, 31^3 99 -> 20, 255x31x15 107 -> 44: faster
-            // at every size; contiguous lines need 16-byte aligned arrays
+            // 255^3 462 -> 213 us a solve, 127^3 96 -> 60, 31^3 99 -> 20; not for few lines of 255
+            // samples, and contiguous lines need 16-byte aligned arrays
             if (dst_lines(lm, a == 1, out, in, lines, n_inner, s_inner, s_outer, step, c,
                           (const T*)sc.lam_q, (const T*)sc.lam_r, (const T*)sc.lam_s, sc.lam_div, reps, s)) {
                 hipError_t e = done("dst_lines_kernel");
