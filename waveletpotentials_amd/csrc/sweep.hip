@@ -329,6 +329,28 @@ constexpr int kStripMax = sizeof(T) == 8 ? 256 : 320;
 template <class T>
 int strips(int outputs) { return (outputs + kStrip<T> - 1) / kStrip<T>; }
 
+// Which kernel transforms `lines` lines of n samples, n + 1 not a power of two up to
+// 1024.  Strided lines: the strips, up to their longest line (faster than the tiled
+// product at every count measured, 225 to 65025 lines).  Contiguous lines touch 64
+// lines of memory per load, which the L1 holds for a while only: from memory up to 2^20
+// samples (FP64 lines of 160 and more, whose 64 take 82 KB: 2^19).  Above that the tiled
+// product, and where 64 lines fit LDS twice, the line count fills the chip with
+// workgroups of 64 and (FP32) the tiled product is not yet short of memory instead, the
+// rows in LDS.  us a solve with two passes over those lines, tiled / strips / rows: FP32
+// 3969 lines of 100 70 / 53 / 62, of 256 119 / 107 / 168, of 300 165 / 170 / 230; 8001 of 200
+// 141 / 161 / 151; 16129 of 80 88 / 95 / 79, of 200 181 / 264 / 169, of 256 194 / 338 / 206; 65025 of
+// 100 216 / 294 / 223, of 200 464 / 1006 / 543.  FP64 3969 of 100 106 / 78 / 106, of 160 146 / 159,
+// of 256 203 / 206; 16129 of 100 182 / 183 / 159, of 256 394 / 670; 65025 of 80 418 / 534 / 403.
+enum DstKernel { kDstTiled, kDstStrips, kDstRows };
+template <class T>
+DstKernel dst_kernel_of(int n, int64_t lines, bool contig) {
+    if (n > kStripMax<T>) return kDstTiled;
+    constexpr bool f64 = sizeof(T) == 8;
+    if (!contig || lines * n <= (f64 && n >= 160 ? 1 << 19 : 1 << 20)) return kDstStrips;
+    const bool fits = 2 * 64 * (size_t)(n | 1) * sizeof(T) <= kMaxLdsBytes;
+    return fits && lines >= 12288 && (f64 || (n <= 220 && lines <= 24576)) ? kDstRows : kDstTiled;
+}
+
 template <class T>
 __global__ void __launch_bounds__(256) dst_strip_kernel(T* __restrict__ out, const T* __restrict__ in,
                                                         const T* __restrict__ S, int n, int64_t lines, int m,
@@ -391,9 +413,7 @@ __global__ void __launch_bounds__(256) dst_strip_kernel(T* __restrict__ out, con
 // The strips of contiguous lines (the y axis) in one workgroup per 64 lines: the
 // lines are one block of memory, staged in LDS (rows of n | 1 values, so the
 // lanes' walks hit every bank once), and the outputs go back through LDS the same
-// way.  Lane by lane from memory every load and store touches 64 lines of it: from
-// 2^20 samples this is the faster one (a 120^3 FP64 solve 169 -> 151 us, FP32 153 ->
-// 128; 49^3 37 -> 44 and 48 -> 54, where its second barrier and copy weigh more).
+// way.  dst_kernel_of says where this is the fastest of the three.
 template <class T>
 __global__ void __launch_bounds__(1024) dst_strip_rows_kernel(T* __restrict__ out, const T* __restrict__ in, const T* __restrict__ S,
                                       int n, int64_t lines) {
@@ -883,18 +903,20 @@ int dst_pass(const whhd_dst3d_s* h, T* out, const T* in, int a, hipStream_t s,
         hipError_t e = done("dst_fft_kernel");
         return e == hipSuccess ? WHHD_OK : hip_fail(e, "dst fft kernel");
     }
-    if (n <= kStripMax<T>) {
-        const int64_t lines = (int64_t)m * nb;
+    const int64_t lines = (int64_t)m * nb;
+    const DstKernel kernel = dst_kernel_of<T>(n, lines, a == 1);
+    if (kernel == kDstRows) {
+        const int all = strips<T>((n + 1) / 2) + strips<T>(n / 2);
+        hipLaunchKernelGGL(dst_strip_rows_kernel<T>, dim3((unsigned)((lines + 63) / 64)),
+                           dim3(64 * std::min(all, 16)), 2 * 64 * (size_t)(n | 1) * sizeof(T), s, out, in,
+                           (const T*)h->S[a], n, lines);
+        hipError_t e = done("dst_strip_rows_kernel");
+        return e == hipSuccess ? WHHD_OK : hip_fail(e, "dst strip rows kernel");
+    }
+    if (kernel == kDstStrips) {
         const int all = strips<T>((n + 1) / 2) + strips<T>(n / 2);
         // lines of the z pass are li = y + x n2
         const T* const none = nullptr;
-        const size_t rows_lds = 2 * 64 * (size_t)(n | 1) * sizeof(T);
-        if (sj == 1 && rows_lds <= kMaxLdsBytes && !scale && lines * n >= 1 << 20) {
-            hipLaunchKernelGGL(dst_strip_rows_kernel<T>, dim3((unsigned)((lines + 63) / 64)),
-                               dim3(64 * std::min(all, 16)), rows_lds, s, out, in, (const T*)h->S[a], n, lines);
-            hipError_t e = done("dst_strip_rows_kernel");
-            return e == hipSuccess ? WHHD_OK : hip_fail(e, "dst strip rows kernel");
-        }
         hipLaunchKernelGGL(dst_strip_kernel<T>, dim3((unsigned)((lines + 63) / 64), (all + 3) / 4), dim3(256), 0,
                            s, out, in, (const T*)h->S[a], n, lines, m, si, sj, sb,
                            scale ? (const T*)h->lam[0] : none, scale ? (const T*)h->lam[1] : none,
@@ -955,7 +977,8 @@ int dst3d_create_t(int n1, int n2, int n3, double dx, double dy, double dz, bool
             auto sine = [&](int k, int j) {
                 return sc * std::sin(M_PI * (double)((int64_t)(k + 1) * (j + 1) % (2 * (n + 1))) / (n + 1));
             };
-            if (n <= kStripMax<T>) {
+            // the strips' table or the dense one, as dst_pass picks the kernel
+            if (dst_kernel_of<T>(n, (int64_t)n1 * n2 * n3 / n, a == 1) != kDstTiled) {
                 const int rows = (n + 1) / 2, even = strips<T>(rows) * kStrip<T>;
                 const int pitch = even + strips<T>(n / 2) * kStrip<T>;
                 S.assign((size_t)rows * pitch, T(0));
