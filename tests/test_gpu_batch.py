@@ -17,7 +17,7 @@ from waveletpotentials_amd import inputs as I
 
 pytestmark = pytest.mark.gpu
 
-# sizes below 32 cells run the windowed kernels one problem at a time
+# sizes down to 8 cells an axis, the smallest of the line-parallel kernels
 DIMS = [(32, 32, 32), (64, 32, 32), (32, 32, 32), (16, 16, 16), (32, 64, 32), (64, 32, 32),
         (32, 32, 32), (8, 8, 8), (32, 32, 64)]
 
@@ -77,7 +77,7 @@ def test_batch_equals_single_solves(whhd, kernel_mode):
 
 
 def test_batch_velocity_bc_d_equals_single_solves(whhd):
-    """Velocity bc 'd' runs the windowed transforms and the divergence bc 'n'
+    """Velocity bc 'd': the other wavelet pair's kernels and the divergence bc 'n'
     projection per size class; still bit for bit the single-grid solves."""
     dims = [(32, 32, 32), (16, 16, 16), (32, 32, 32), (16, 32, 8)]
     b = make(whhd, dims, "d")
@@ -88,6 +88,26 @@ def test_batch_velocity_bc_d_equals_single_solves(whhd):
         ref = single(whhd, d, b.arrays(i), "d")
         for g, r in zip(got[i], ref):
             assert torch.equal(g, r), f"problem {i} {d} differs from the single-grid solve"
+
+
+def test_groups_of_a_large_class_equal_single_solves(whhd):
+    """Ten problems of 128^3: a class is solved in groups of at most 68 MB a component
+    (eight of these), so the last two are a group of their own.  White noise: the
+    solve of any velocity has to be the single-grid one bit for bit."""
+    dims = [(128, 128, 128)] * 10
+    b = make(whhd, dims)
+    g = torch.Generator(device="cpu").manual_seed(9)
+    for i in range(len(dims)):
+        a = b.arrays(i)
+        for k in ("xv", "yv", "zv"):
+            a[k].copy_(torch.randn(a[k].shape, generator=g))
+        for k in ("qx", "qy", "qz"):
+            a[k].fill_(float("nan"))
+    b.Solve()
+    for i in (0, 7, 8, 9):
+        a = b.arrays(i)
+        for k, r in zip(("qx", "qy", "qz"), single(whhd, dims[i], a)):
+            assert torch.equal(a[k], r), (i, k)
 
 
 def test_batch_problem_matches_oracle(whhd, orc):
