@@ -3,8 +3,8 @@ relaxations of every tile, whatever the count.
 
 A call of few relaxations runs every tile, so a long run must equal the same number
 of relaxations taken seven at a time.  Tiles are 64 y x 4 x x 4 or 8 z, eight on
-grids of at least 2048 of those: extents around both with remainders, axes of one
-cell, values beyond the 1e8 that stands for the outside, infinities and NaN; and an
+grids of at least 2048 of those, and one or two planes deep on grids that are: extents
+around them with remainders, axes of one cell, values beyond the 1e8 that stands for the outside, infinities and NaN; and an
 array of 2^31 bytes and more, whose offsets are 64-bit, against a narrow copy of it
 whose are not.  The eight-plane tiles are held against the FP64 oracle too, at the
 2e-6 of the solid-geometry tests.
@@ -26,7 +26,8 @@ def relax(whhd, ls, n, h, iters):
 
 
 @pytest.mark.parametrize("n", [(8, 64, 32), (9, 65, 33), (70, 130, 50), (1, 40, 20), (30, 1, 40),
-                               (20, 50, 1), (70, 321, 150), (129, 130, 170)])
+                               (20, 50, 1), (70, 321, 150), (129, 130, 170),
+                               (1030, 1020, 1), (730, 720, 2)])
 @pytest.mark.parametrize("special", [False, True])
 def test_skipped_tiles_equal_every_tile(whhd, n, special):
     nx, ny, nz = n
@@ -80,3 +81,38 @@ def test_64_bit_offsets(whhd):
     torch.cuda.synchronize()
     for k in range(0, n, 20):
         assert torch.equal(wide[k:k + 20].view(torch.int32), narrow[k:k + 20, :1].view(torch.int32).expand(20, n, n)), k
+
+
+def test_long_run_beside_a_capture(whhd):
+    """A run that leaves tiles out takes memory from its stream's pool: on a stream of
+    its own while another one is being captured, and in a captured stream itself,
+    where every tile runs.  The capture stays valid and all results agree."""
+    n = (40, 70, 30)
+    h = 1.0 / 70
+    g = torch.Generator(device="cpu").manual_seed(4)
+    ls = torch.rand((30, 40, 70), generator=g).cuda() - 0.2
+    want = ls.clone()
+    for _ in range(16):
+        relax(whhd, want, n, h, 7)
+    beside, inside, x = ls.clone(), ls.clone(), torch.ones(1000, device="cuda")
+    scratch = [torch.empty_like(ls), torch.empty_like(ls)]
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+
+    def run(t, k, stream):
+        assert whhd.lib().whhd_eikonal_sweep(t.data_ptr(), scratch[k].data_ptr(), *n, ctypes.c_double(h), 112,
+                                             ctypes.c_void_p(stream.cuda_stream)) == 0
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.mul_(2.0)
+        run(beside, 0, other)
+        run(inside, 1, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    assert torch.equal(beside, want)
+    for k in range(3):
+        inside.copy_(ls)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(inside, want)
+        assert float(x[0]) == 2.0 ** (k + 1)

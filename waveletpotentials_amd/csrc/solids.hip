@@ -10,6 +10,7 @@
 // faces near the interface (16384 samples each) and streaming elsewhere.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
@@ -122,11 +123,9 @@ __device__ __forceinline__ float eikonal_update(float a, float b, float c, float
 // chg_out[tile] receives this one's.  The field settles outwards from the solids
 // (a cell depends on smaller neighbours only), long before the 1.5-2 max(n)
 // relaxations that a caller asks for to be sure.
-// 320 relaxations of 160x120x136: 3.59 -> 1.84 ms (2.49 with a load behind every
-// store), 384 of 192^3: 6.31 -> 3.53.
-//
-// kEikZ: 8, or 4 on grids that would give fewer than 512 workgroups (64x48x40: 4
-// 3.1 us a relaxation, 8 3.6; 160x120x136: 4 6.0, 8 5.8, 16 8.5).
+// 320 relaxations of 160x120x136: 3.57 -> 1.84 ms, 384 of 192^3: 6.29 -> 3.97, 1024 of
+// 512^3: 286 -> 137.  (With the column walked plane by plane, a load behind every store,
+// 160x120x136 took 12.0 us a relaxation, with the loads ahead 8.8, 512^3 279 and 258.)
 template <class I, int kEikZ>
 __global__ void __launch_bounds__(256) eikonal_kernel(float* __restrict__ dst, const float* __restrict__ src,
                                                       int nx, int ny, int nz, float h,
@@ -135,13 +134,11 @@ __global__ void __launch_bounds__(256) eikonal_kernel(float* __restrict__ dst, c
     const unsigned gx = gridDim.x, gy = gridDim.y;
     const unsigned tile = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
     if (chg_in) {
-        int any = chg_in[tile];
-        if (blockIdx.x > 0) any |= chg_in[tile - 1];
-        if (blockIdx.x + 1 < gx) any |= chg_in[tile + 1];
-        if (blockIdx.y > 0) any |= chg_in[tile - gx];
-        if (blockIdx.y + 1 < gy) any |= chg_in[tile + gx];
-        if (blockIdx.z > 0) any |= chg_in[tile - gx * gy];
-        if (blockIdx.z + 1 < gridDim.z) any |= chg_in[tile + gx * gy];
+        // all seven in flight together; a neighbour outside the grid is the tile itself
+        const unsigned tx = blockIdx.x, ty = blockIdx.y, tz = blockIdx.z, g = gx * gy;
+        const int any = chg_in[tile] | chg_in[tx > 0 ? tile - 1 : tile] | chg_in[tx + 1 < gx ? tile + 1 : tile] |
+                        chg_in[ty > 0 ? tile - gx : tile] | chg_in[ty + 1 < gy ? tile + gx : tile] |
+                        chg_in[tz > 0 ? tile - g : tile] | chg_in[tz + 1 < gridDim.z ? tile + g : tile];
         if (!any) {
             if (threadIdx.x == 0 && threadIdx.y == 0) chg_out[tile] = 0;
             return;
@@ -409,14 +406,28 @@ int eikonal_sweep(float* ls, float* scratch, int nx, int ny, int nz, double h, i
     float* a = ls;
     float* b = scratch;
     const int64_t columns = (int64_t)((ny + 63) / 64) * ((nx + 3) / 4);
-    const int zb = columns * ((nz + 7) / 8) < 512 ? 4 : 8;
+    // Planes a tile: four; eight where that leaves 2048 workgroups or more (us a
+    // relaxation by four / eight: 64x48x40 3.7 / 4.4, 160x120x136 8.8 / 10.1, 192^3 16.1 / 16.4
+    // and, with tiles left out, 384 relaxations 4149 / 3992, 512^3 1024 relaxations 155 / 137
+    // ms), unless half of the last eight planes of a shallow grid would lie outside it
+    // (1024x1024x9 21.1 / 22.3); grids of one and two planes their own depth
+    // (1024x1024x1 by one 6.5, by four 7.3).
+    const int r8 = nz & 7;
+    const bool deep = nz > 4 && (r8 == 0 || r8 > 4 || nz >= 32) && columns * ((nz + 7) / 8) >= 2048;
+    const int zb = nz < 3 ? nz : deep ? 8 : 4;
     const dim3 grid((ny + 63) / 64, (nx + 3) / 4, (nz + zb - 1) / zb);
     const size_t tiles = (size_t)grid.x * grid.y * grid.z;
-    // two sets of tile flags from the stream's memory pool; without them (few
-    // relaxations, a stream being captured, no memory) every tile runs
+    // Two sets of tile flags from the stream's memory pool, where leaving tiles out
+    // pays: the allocation takes 20 us of the host, the flags about a tenth of a
+    // relaxation, and what settles in a call of fewer relaxations than the grid's
+    // longest side is little (us, all tiles / flags: 256x256x2 8 relaxations 28 / 49,
+    // 1024x1024x4 40 402 / 531, 192^3 96 1504 / 1689, 192 3140 / 2998).  Small grids of one
+    // or two planes are bound by their launches (300x200x1 600 1637 / 1895).  Without
+    // flags (also in a stream being captured, or without memory) every tile runs.
     uint8_t* flags = nullptr;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (n_iters >= 8) {
+    if (n_iters >= std::max(64, std::max(nx, std::max(ny, nz))) &&
+        (nz > 2 || (int64_t)nx * ny * nz >= (int64_t)1 << 20)) {
         const hipError_t e = hipStreamIsCapturing(s, &cap);
         if (e == hipSuccess && cap == hipStreamCaptureStatusNone &&
             hipMallocAsync((void**)&flags, 2 * tiles, s) != hipSuccess) {
@@ -429,12 +440,15 @@ int eikonal_sweep(float* ls, float* scratch, int nx, int ny, int nz, double h, i
     for (int i = 0; i < n_iters; ++i) {
         const uint8_t* in = flags && i > 0 ? flags + (i & 1) * tiles : nullptr;
         uint8_t* out = flags ? flags + (1 - (i & 1)) * tiles : nullptr;
-        if (wide)
-            hipLaunchKernelGGL((eikonal_kernel<int64_t, 8>), grid, dim3(64, 4), 0, s, b, a, nx, ny, nz, (float)h, in, out);
-        else if (zb == 8)
-            hipLaunchKernelGGL((eikonal_kernel<int, 8>), grid, dim3(64, 4), 0, s, b, a, nx, ny, nz, (float)h, in, out);
-        else
-            hipLaunchKernelGGL((eikonal_kernel<int, 4>), grid, dim3(64, 4), 0, s, b, a, nx, ny, nz, (float)h, in, out);
+#define WHHD_EIK(ZB)                                                                                       \
+    case ZB:                                                                                               \
+        if (wide) hipLaunchKernelGGL((eikonal_kernel<int64_t, ZB>), grid, dim3(64, 4), 0, s, b, a, nx, ny, \
+                                     nz, (float)h, in, out);                                               \
+        else hipLaunchKernelGGL((eikonal_kernel<int, ZB>), grid, dim3(64, 4), 0, s, b, a, nx, ny, nz,      \
+                                (float)h, in, out);                                                        \
+        break;
+        switch (zb) { WHHD_EIK(1) WHHD_EIK(2) WHHD_EIK(4) WHHD_EIK(8) }
+#undef WHHD_EIK
         float* t = a;
         a = b;
         b = t;
