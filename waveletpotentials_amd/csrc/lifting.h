@@ -438,23 +438,28 @@ struct Wavelet {
     static constexpr const double* il10 = IL10;
 };
 
-// y = M x over lanes 0..M-1 (lane r gets row r); other lanes return row 0.
-// The row is selected from scalar loads of the whole matrix.  A row loaded by each
-// lane instead is faster for a few lines (2D recovery of 128^2 23.8 against 24.2 us)
-// but slower for many short ones (16384 strided lines of 4 samples 5.3 against 4.5 us)
-// and for long strided ones (4096 samples 26 against 24).
+// y = M x over lanes 0..M-1 (lane r gets row r); other lanes return row 0.  A lane's
+// row is loaded once for all the lines its wavefront lifts: M loads in flight together.
+// us, row selected from scalar loads of the whole matrix in every line / loaded in every
+// line / once: 16384 strided FP64 lines of 8 samples, inverse, 13.4 / 10.7 / 10.6; FP32 of 4
+// samples, forward, 4.5 / 5.4 / 4.4; one FP32 line of 4096 samples 24 / 26 / 25.
+template <int M, class T>
+struct L10Row {
+    T c[M];
+};
 template <int M, const double* Mat, class T>
-WHHD_DEV T apply_l10(T v, int lane) {
-    const int r = lane < M ? lane : 0;
+WHHD_DEV L10Row<M, T> l10_row(int lane) {
+    const double* row = Mat + (lane < M ? lane : 0) * M;
+    L10Row<M, T> r;
+#pragma unroll
+    for (int c = 0; c < M; ++c) r.c[c] = T(row[c]);
+    return r;
+}
+template <int M, class T>
+WHHD_DEV T apply_l10(const L10Row<M, T>& row, T v) {
     T acc = T(0);
 #pragma unroll
-    for (int c = 0; c < M; ++c) {
-        T xc = lane_get(v, c);
-        T coef = T(0);
-#pragma unroll
-        for (int rr = 0; rr < M; ++rr) coef = (r == rr) ? T(Mat[rr * M + c]) : coef;
-        acc += xc * coef;
-    }
+    for (int c = 0; c < M; ++c) acc += lane_get(v, c) * row.c[c];
     return acc;
 }
 

@@ -36,7 +36,7 @@ WHHD_DEV void lds_order() { asm volatile("" ::: "memory"); }
 // details of level l go to r[2^l+ext, 2^(l+1)+ext), the last 4+ext
 // approximations get the dense L10 matrix.
 template <class W, class T>
-WHHD_DEV void forward_line(T* s, T* r, int n, int levels, int lane) {
+WHHD_DEV void forward_line(T* s, T* r, int n, int levels, int lane, const L10Row<W::m10, T>& l10) {
     constexpr int H = W::halo;
     constexpr int WL = kWave - 2 * H;
     const int ext = n & 1;
@@ -71,7 +71,7 @@ WHHD_DEV void forward_line(T* s, T* r, int n, int levels, int lane) {
     } else {
         if (lane < W::m10) a = s[lane];
     }
-    const T v = apply_l10<W::m10, W::l10>(a, lane);
+    const T v = apply_l10(l10, a);
     if (lane < W::m10) r[lane] = v;
     lds_order();
 }
@@ -83,7 +83,7 @@ WHHD_DEV void forward_line(T* s, T* r, int n, int levels, int lane) {
 // input buffer is reused once its details have been consumed.  Returns the
 // buffer holding the result.
 template <class W, class T>
-WHHD_DEV T* inverse_line(T* in, T* other, int n, int levels, int lane) {
+WHHD_DEV T* inverse_line(T* in, T* other, int n, int levels, int lane, const L10Row<W::m10, T>& l10) {
     constexpr int H = W::halo;
     constexpr int WL = kWave - 2 * H;
     const int ext = n & 1;
@@ -95,7 +95,7 @@ WHHD_DEV T* inverse_line(T* in, T* other, int n, int levels, int lane) {
     }
     T a = T(0), d = T(0);
     if (lane < W::m10) a = in[lane];
-    const T v = apply_l10<W::m10, W::il10>(a, lane);
+    const T v = apply_l10(l10, a);
     lds_order();
     if (lane < W::m10) dst[lane] = v;
     lds_order();
@@ -182,11 +182,12 @@ WHHD_DEV void line_tile(T* dst, const T* src, const LineGeom& g, unsigned tile_i
     // Both directions leave every line's result in buf1: the forward writes its
     // outputs there, and the inverse starts its ping-pong so that the last
     // level lands in the second buffer whatever the level count.
+    const L10Row<W::m10, T> l10 = l10_row<W::m10, FWD ? W::l10 : W::il10, T>(lane);
     for (int li = wave; li < lines_here; li += nwaves) {
         T* s = buf0 + li * ls;
         T* r = buf1 + li * ls;
-        if (FWD) forward_line<W, T>(s, r, n, g.levels, lane);
-        else inverse_line<W, T>(s, r, n, g.levels, lane);
+        if (FWD) forward_line<W, T>(s, r, n, g.levels, lane, l10);
+        else inverse_line<W, T>(s, r, n, g.levels, lane, l10);
     }
     __syncthreads();
 
