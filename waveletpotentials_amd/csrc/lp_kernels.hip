@@ -47,7 +47,7 @@ bool lp_interleaves(int wt_curl, char bc_curl, int wt_div, char bc_div, int leve
 // read ahead of its stores: the inverse, and either direction interleaved.
 int lp_transform(const LineJob* jobs, int njobs, int levels, char axis, bool fwd, bool interleaved,
                  hipStream_t stream, int waves, int nb) {
-    if (njobs < 1 || njobs > lp::kMaxJobs) return -1;
+    if (njobs < 1 || njobs > lp::kMaxJobs || levels < 3 || levels > 8) return -1;
     lp::LpJobs a{};
     a.n = njobs;
     int pair = -1;
