@@ -1242,10 +1242,14 @@ int mgfrac3d_create(const float* ax, const float* ay, const float* az, int nx, i
         L.ax = (float*)alloc((size_t)(d.x + 1) * d.y * d.z * 4);
         L.ay = (float*)alloc((size_t)d.x * (d.y + 1) * d.z * 4);
         L.az = (float*)alloc((size_t)d.x * d.y * (d.z + 1) * 4);
-        L.hx = (float*)alloc((size_t)d.x * 4);
-        L.hy = (float*)alloc((size_t)d.y * 4);
-        L.hz = (float*)alloc((size_t)d.z * 4);
-        if (!L.f || !L.v || !L.t || !L.ax || !L.ay || !L.az || !L.hx || !L.hy || !L.hz) {
+        // spacings and face factors
+        L.hx = (float*)alloc((size_t)3 * (d.x + d.y + d.z) * 4);
+        if (L.hx) {
+            L.hy = L.hx + d.x;
+            L.hz = L.hy + d.y;
+            L.kf = L.hz + d.z;
+        }
+        if (!L.f || !L.v || !L.t || !L.ax || !L.ay || !L.az || !L.hx) {
             st = fail(WHHD_OOM, "mgfrac3d_create: allocation failed");
             break;
         }
@@ -1310,11 +1314,6 @@ int mgfrac3d_create(const float* ax, const float* ay, const float* az, int nx, i
     for (Level& L : h->lv) {
         if (st != WHHD_OK) break;
         const int nk = 2 * (L.d.x + L.d.y + L.d.z);
-        L.kf = (float*)alloc((size_t)nk * 4);
-        if (!L.kf) {
-            st = fail(WHHD_OOM, "mgfrac3d_create: allocation failed");
-            break;
-        }
         hipLaunchKernelGGL(face_factor_kernel, dim3((nk + 255) / 256), dim3(256), 0, s, L.kf, L.hx, L.hy,
                            L.hz, L.d.x, L.d.y, L.d.z, h->he[0], h->he[1], h->he[2]);
         hipError_t e = launch_status("mg_face_factor_kernel");
