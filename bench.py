@@ -74,25 +74,34 @@ def stage_bytes(stage, ab):
     return 2 * ab[stage.split()[1]]
 
 
-def measured_traffic(kernel):
-    """HBM bytes per launch of `kernel` from the committed rocprof counter
+def measured_traffic(kernel, algorithmic_bytes):
+    """Memory bytes per launch of `kernel` from the committed rocprof counter
     summary (FETCH_SIZE and WRITE_SIZE runs, each scaled by the calibration
     kernel's reading), or None when the summary does not cover it.  The summary
     lists a line-parallel kernel with both wavelets of its pair and names the
-    strided kernel that writes the interleaved order apart."""
+    strided kernel that writes the interleaved order apart.  A line-parallel kernel
+    runs both on one array (a traced solve) and on the three components together: the
+    launch of one array, a work-item per line, is the one of `algorithmic_bytes`."""
     path = os.path.join(ROOT, "profiles", "traffic_recover3d_256.json")
     try:
         with open(path) as f:
             rows = json.load(f)
     except (OSError, ValueError):
         return None
-    kernels = rows.get("kernels", {})
-    row = kernels.get(kernel)
-    m = re.match(r"lp_kernel<([^,]+),(.*)>$", kernel)
-    for name, r in kernels.items() if m and not row else ():
-        k = re.match(r"lp_kernel<([^,]+),(.*)>$", name)
-        if k and m.group(1) in k.group(1).split(" + ") and k.group(2).replace("interleaved", "strided") == m.group(2):
-            row = r
+    row = rows.get("kernels", {}).get(kernel)
+    m = re.match(r"lp_kernel<([^,]+),L=(\d+),(\w+),(\w+)>$", kernel)
+    if m:
+        wavelet, levels, way, layout = m.groups()
+        samples = (1 << int(levels)) + wavelet.startswith("cdf4")
+        lines = algorithmic_bytes / 8 / samples
+        row = None
+        for r in rows.get("by_size", []):
+            k = re.match(r"lp_kernel<([^,]+),L=(\d+),(\w+),(\w+)>$", r["kernel"])
+            if (k and wavelet in k.group(1).split(" + ") and k.group(2, 3) == (levels, way)
+                    and k.group(4).replace("interleaved", "strided") == layout
+                    and abs(r["grid"] - lines) <= 0.02 * lines
+                    and (row is None or abs(r["grid"] - lines) < abs(row["grid"] - lines))):
+                row = r
     if not row:
         return None
     return {"bytes": int(row["fetch_bytes"] + row["write_bytes"]),
@@ -177,7 +186,7 @@ def main():
     dom_us = dom["us"] / dom["launches"]
     dom_bytes = dom["bytes"] / dom["launches"]
     achieved = dom_bytes / (dom_us * 1e-6) / 1e9
-    traffic = measured_traffic(dom_name)
+    traffic = measured_traffic(dom_name, dom_bytes)
 
     out = {
         "metric": METRIC,
@@ -200,6 +209,8 @@ def main():
                      "kernel": dom_name, "launches_per_solve": dom["launches"],
                      "algorithmic_bytes_per_launch": int(dom_bytes),
                      "avg_launch_us": round(dom_us, 2),
+                     "launches": "of a traced solve, one array each; a timed solve launches the "
+                                 "three components of a pass together",
                      "traffic_source": traffic["source"] if traffic else None},
         "stage_model": {"bytes_per_solve": int(bytes_per_solve),
                         "solve_GBs": round(bytes_per_solve / (ms_per_step * 1e-3) / 1e9, 1),

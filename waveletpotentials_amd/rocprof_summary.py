@@ -9,8 +9,9 @@ bench.py runs on a known size (an elementwise multiply reading and writing
     python -m waveletpotentials_amd.rocprof_summary TRACE_DIR FETCH_DIR WRITE_DIR OUT_PREFIX \\
         --command "..."
 
-writes OUT_PREFIX.md (per-kernel durations and bytes) and OUT_PREFIX.json
-(per-kernel fetch/write bytes, read by bench.py for ``roofline.traffic``).
+writes OUT_PREFIX.md (per-kernel durations and bytes, means over the launches) and
+OUT_PREFIX.json (the same numbers, and those of every launch size of a kernel that has
+several, read by bench.py for ``roofline.traffic``).
 With ``--trace-only TRACE_DIR OUT_PREFIX`` it writes OUT_PREFIX.md with the
 per-kernel durations of one ``--kernel-trace --stats`` run.
 """
@@ -115,12 +116,15 @@ def summarize(trace_dir, fetch_dir, write_dir):
         row = kernels.setdefault(label, {"calls": 0, "total_ns": 0.0, "library": is_library(name)})
         row["calls"] += int(r["Calls"])
         row["total_ns"] += float(r["TotalDurationNs"])
-        if name in fetch:
-            row["fetch_bytes"] = statistics.median(fetch[name]) * f_scale
-        if name in write:
-            row["write_bytes"] = statistics.median(write[name]) * w_scale
+        # means, as the durations are: a kernel may be launched at several sizes
+        for key, runs, scale in (("fetch_bytes", fetch, f_scale), ("write_bytes", write, w_scale)):
+            if name in runs:
+                row[key] = row.get(key, 0.0) + statistics.mean(runs[name]) * scale * int(r["Calls"])
     for row in kernels.values():
         row["avg_us"] = row["total_ns"] / row["calls"] / 1000.0
+        for key in ("fetch_bytes", "write_bytes"):
+            if key in row:
+                row[key] /= row["calls"]
     # library kernels launched at several sizes (one per multigrid level, say):
     # one row per launch size
     durs = durations_by_grid(trace_dir)
@@ -135,9 +139,9 @@ def summarize(trace_dir, fetch_dir, write_dir):
         row = {"kernel": kernel_label(name), "grid": g, "calls": len(d),
                "avg_us": statistics.mean(d) / 1000.0}
         if (name, g) in fg:
-            row["fetch_bytes"] = statistics.median(fg[(name, g)]) * f_scale
+            row["fetch_bytes"] = statistics.mean(fg[(name, g)]) * f_scale
         if (name, g) in wg:
-            row["write_bytes"] = statistics.median(wg[(name, g)]) * w_scale
+            row["write_bytes"] = statistics.mean(wg[(name, g)]) * w_scale
         by_size.append(row)
     by_size.sort(key=lambda r: (r["kernel"], -r["grid"]))
     return kernels, f_scale, w_scale, by_size
@@ -150,12 +154,19 @@ def write_outputs(kernels, f_scale, w_scale, prefix, command, by_size=()):
                    "kernels": {k: {"avg_us": round(v["avg_us"], 3), "calls": v["calls"],
                                    "fetch_bytes": round(v.get("fetch_bytes", 0.0)),
                                    "write_bytes": round(v.get("write_bytes", 0.0))}
-                               for k, v in sorted(lib.items())}}, f, indent=1)
+                               for k, v in sorted(lib.items())},
+                   "by_size": [{"kernel": v["kernel"], "grid": v["grid"], "calls": v["calls"],
+                                "avg_us": round(v["avg_us"], 3),
+                                "fetch_bytes": round(v.get("fetch_bytes", 0.0)),
+                                "write_bytes": round(v.get("write_bytes", 0.0))}
+                               for v in by_size]}, f, indent=1)
     lines = [f"# rocprofv3 summary: {os.path.basename(prefix)}", "",
              "Command (three runs; byte counters scaled by the calibration kernel, "
              f"FETCH_SIZE x{f_scale:.3f}, WRITE_SIZE x{w_scale:.3f}):", "", "```", command, "```",
-             "", "HBM GB/s = (fetch + write bytes) / average duration; peak 8000 GB/s.", "",
-             "| kernel | calls | avg us | HBM fetch MB/launch | HBM write MB/launch | HBM GB/s | % of peak |",
+             "", "Bytes and durations are means over a kernel's launches of all sizes; the counters are",
+             "at the L2's memory side, so the bytes include what the Infinity Cache serves.",
+             "GB/s = (fetch + write bytes) / average duration; peak 8000 GB/s.", "",
+             "| kernel | calls | avg us | fetch MB/launch | write MB/launch | GB/s | % of peak |",
              "|---|---:|---:|---:|---:|---:|---:|"]
     for k, v in sorted(lib.items(), key=lambda kv: -kv[1]["total_ns"]):
         b = v.get("fetch_bytes", 0) + v.get("write_bytes", 0)
@@ -165,7 +176,7 @@ def write_outputs(kernels, f_scale, w_scale, prefix, command, by_size=()):
                      f"{gbs:.0f} | {100 * gbs / 8000:.1f}% |")
     if by_size:
         lines += ["", "Kernels launched at several sizes, one row per launch size (work-items):", "",
-                  "| kernel | work-items | calls | avg us | HBM fetch MB/launch | HBM write MB/launch | HBM GB/s | % of peak |",
+                  "| kernel | work-items | calls | avg us | fetch MB/launch | write MB/launch | GB/s | % of peak |",
                   "|---|---:|---:|---:|---:|---:|---:|---:|"]
         for v in by_size:
             b = v.get("fetch_bytes", 0) + v.get("write_bytes", 0)
