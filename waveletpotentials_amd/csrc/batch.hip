@@ -4,8 +4,9 @@
 // here gets exactly that solve.
 //
 // Problems with equal extents and spacing form a size class.  A class is one
-// recovery driver over its problems stored back to back, so each of its 19
-// stages is one launch whose grid rows are the problems.  Classes are
+// recovery driver over its problems stored back to back, so each of its stages
+// (seven in place, the components of a pass together; 19 array by array) is one launch
+// whose grid rows are the problems, or a group of them (recover.hip).  Classes are
 // independent and run as parallel branches: the first on the given stream, the
 // others on internal streams forked from it and joined back with events.
 // Captured once, the whole batch is one hipGraph replayed by a single call.

@@ -7,14 +7,14 @@
 // potential's own axis uses the curl wavelet and the other axes the
 // divergence wavelet.  The handle owns its scratch (per component one
 // velocity-sized array and one array of the larger of the velocity and the
-// potential sizes, allocated at create: passes run out of place) and enqueues
-// everything on the caller's stream without synchronizing, so a solve can be
-// captured in a HIP graph.
+// potential sizes, allocated at create) and enqueues everything on the caller's
+// stream without synchronizing, so a solve can be captured in a HIP graph.
 //
 // The x and z passes keep every coefficient at the position of the sample it
 // replaces (interleaved order), so that only the first forward pass writes
 // another array than it reads; the projection takes its coefficient rows in
-// that order.
+// that order.  Lengths and wavelets without such kernels are solved array by
+// array and out of place (solve_chains).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -48,9 +48,11 @@ struct whhd_recover3d_s {
     int lp_waves_y = 1;  // the y (contiguous) passes: 0.691 ms against 0.695 with 2
     whhd_project3d_s* proj = nullptr;
     float* tmp[3] = {nullptr, nullptr, nullptr};  // transformed velocity (velocity-sized)
-    // ping-pong scratch of component c: the potential's coefficients and the
-    // middle pass of both of component c's three-pass chains, so it holds
-    // max(velocity size, potential size) elements per problem
+    // ping-pong scratch of component c out of place: the potential's coefficients
+    // and the middle pass of both of component c's three-pass chains, so it holds
+    // max(velocity size, potential size) elements per problem.  Solves in place do
+    // not touch it, but the level cut does, and so does any handle while the
+    // windowed kernels are chosen, and neither may allocate (stream capture)
     float* sq[3] = {nullptr, nullptr, nullptr};
     size_t sq_elems[3] = {0, 0, 0};  // elements per problem of sq[c]
     whhd::StageTrace trace;
@@ -210,13 +212,14 @@ static int in_place_passes(const whhd_recover3d_s* h, const Chain* ch, int n, co
 // instead of 19 (32^3 72 -> 30 us, 128^3 187 -> 83), three times the wavefronts
 // per launch, and in place the three arrays are the whole working set: up to 67
 // MB each (256^3) it fits the 256 MB Infinity Cache.  256^3: 660 us (out of
-// place, one by one), 627 (in place, one by one), 560 (in place, together);
-// 64 grids of 32^3..128^3 in groups of 17, 34, 68 and 1000 MB: 1.90, 1.90, 1.87
-// and 2.09 ms.
+// place, one by one), 627 (in place, one by one), 560 (in place, together).
+// A batch runs up to four size classes at a time on streams of their own, so what is
+// in flight is several groups, beyond that cache: 64 grids of 32^3..128^3 in groups of
+// 17, 34, 68 and 1000 MB take 1.90, 1.90, 1.87 and 2.09 ms.
 constexpr int64_t kMergeBytes = 68ll << 20;
 
 // Scratch of a recovery handle, elements per problem: tmp[c] holds velocity
-// component c; sq[c] holds potential component c's coefficients and the
+// component c; sq[c], out of place, potential component c's coefficients and the
 // middle pass of velocity c's and potential c's chains.
 void recover3d_scratch_elems(int nx, int ny, int nz, size_t tmp[3], size_t sq[3]) {
     const size_t X = nx, Y = ny, Z = nz;
@@ -427,8 +430,9 @@ int recover2d_solve(whhd_recover2d_s* h, float* qz, const float* xv, const float
     const int X = h->nx, Y = h->ny;
     float* tx = h->tmp[0];
     float* ty = h->tmp[1];
-    // The windowed kernels throughout: a 2D array has too few lines to fill the
-    // chip with a line per lane.
+    // Both components of a forward pass in one launch of the windowed kernels (2D
+    // arrays have too few lines to fill the chip with a line per lane); wavelets that
+    // are no recovery pair one by one.
     const LineJob ax{tx, xv, X + 1, Y, 1, h->bd, h->wd, 0}, bx{ty, yv, X, Y + 1, 1, h->bc, h->wc, 0};
     int r = transform_pair2d(ax, bx, h->lx, 'x', s);
     if (r == -1) {
