@@ -68,29 +68,30 @@ struct ConvOut {
 // CIN + 8 values: the 16 voxels a fragment reads then start in different banks)
 // and every tap reads it there.  The weights come from global memory in
 // fragment order (pack_kernel): 1 KB contiguous per wavefront and chunk.  The
-// wavefronts split the brick's voxel tiles (WM), the channel tiles (WN) and
-// the reduction (KS, summed through LDS at the end): the small grids of the
-// lower levels have few voxels, and what bounds them is the length of a
-// wavefront's chain of chunks, not the matrix cores.  Reading every operand
-// from the caches in each tap, 32 voxels a wavefront, took (48^3 network grid)
-// 14.5 us for 16 -> 16 channels, 41 for 48 -> 16 (48^3), 42 for 96 -> 32 (24^3) and
-// 42 for 64 -> 64 (12^3); this one 7.7, 20, 12 and 10.5.
-template <int CA, int CB, bool UPA, int CO, int MODE, int BZ, int BX, int BY, int WM, int WN, int KS>
-__global__ void __launch_bounds__(64 * WM * WN * KS) conv3_kernel(ConvSrc s, const bf16* __restrict__ w,
+// wavefronts split the brick's voxel tiles (WM) and the channel tiles (WN); every
+// output is summed by one wavefront over the chunks in their order, whatever the
+// split.  The small grids of the lower levels have few voxels, and what bounds them
+// is the number of wavefronts a brick and the chip get, not the matrix cores.
+// Reading every operand from the caches in each tap, 32 voxels a wavefront, took
+// (48^3 network grid) 14.5 us for 16 -> 16 channels, 41 for 48 -> 16 (48^3), 42 for
+// 96 -> 32 (24^3) and 42 for 64 -> 64 (12^3); this one 7.0, 14.6, 12.3 and 5.8.  With the
+// chunks split over wavefronts too and their sums added through LDS (fewer voxel or
+// channel tiles each) the last three took 20, 12.3 and 10.7, and the other order of the
+// sum moved single BF16 activations.
+template <int CA, int CB, bool UPA, int CO, int MODE, int BZ, int BX, int BY, int WM, int WN>
+__global__ void __launch_bounds__(64 * WM * WN) conv3_kernel(ConvSrc s, const bf16* __restrict__ w,
                                                                   ConvOut o) {
     constexpr int CIN = CA + CB;
     static_assert(CIN % 16 == 0 && CA % 8 == 0 && CO % 16 == 0, "channel blocking");
-    constexpr int KC = kpad(CIN) / 32, KCW = (KC + KS - 1) / KS;
+    constexpr int KC = kpad(CIN) / 32;
     constexpr int M = BZ * BX * BY, MT = M / 16, NT = CO / 16, MTW = MT / WM, NTW = NT / WN;
     static_assert(M % 16 == 0 && MT % WM == 0 && NT % WN == 0, "tile split");
     constexpr int HX = BX + 2, HY = BY + 2, HV = (BZ + 2) * HX * HY;
     constexpr int SV = CIN + 8, PV = CIN / 8;
-    constexpr int NTHR = 64 * WM * WN * KS, PIECES = HV * PV, PER = (PIECES + NTHR - 1) / NTHR;
-    constexpr int STAGE = HV * SV + 8;                                // + a zero piece
-    constexpr int RED = KS > 1 ? (KS - 1) * WM * WN * MTW * NTW * 64 * 4 * 2 : 0;  // in bf16 units
-    __shared__ __attribute__((aligned(16))) bf16 sm[STAGE > RED ? STAGE : RED];
+    constexpr int NTHR = 64 * WM * WN, PIECES = HV * PV, PER = (PIECES + NTHR - 1) / NTHR;
+    __shared__ __attribute__((aligned(16))) bf16 sm[HV * SV + 8];  // + a zero piece
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave % WM, wn = (wave / WM) % WN, ks = wave / (WM * WN);
+    const int wm = wave % WM, wn = wave / WM;
     const int m = lane & 15, g = lane >> 4;
     const int by = (s.Y + BY - 1) / BY, bx = (s.X + BX - 1) / BX;
     int bid = blockIdx.x;
@@ -119,11 +120,10 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) conv3_kernel(ConvSrc s, con
         }
     }
     // where the lane's 16 bytes of each chunk lie, relative to its voxel
-    const int k0 = ks * KCW;
-    int off[KCW];
+    int off[KC];
 #pragma unroll
-    for (int i = 0; i < KCW; ++i) {
-        const int k = (k0 + i) * 32 + 8 * g;
+    for (int i = 0; i < KC; ++i) {
+        const int k = i * 32 + 8 * g;
         const int tap = k / CIN, ci = k - tap * CIN;
         off[i] = tap < kTaps ? ((tap / 9 * HX + tap / 3 % 3) * HY + tap % 3) * SV + ci : -1;
     }
@@ -147,39 +147,18 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) conv3_kernel(ConvSrc s, con
         for (int n = 0; n < NTW; ++n) acc[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
     const bf16x8* wf = (const bf16x8*)w + lane;
 #pragma unroll
-    for (int i = 0; i < KCW; ++i) {
-        const int kc = KS > 1 ? min(k0 + i, KC - 1) : i;
+    for (int kc = 0; kc < KC; ++kc) {
         bf16x8 A[NTW];
 #pragma unroll
         for (int n = 0; n < NTW; ++n) A[n] = wf[(int64_t)((wn * NTW + n) * KC + kc) * 64];
 #pragma unroll
         for (int t = 0; t < MTW; ++t) {
             // past the last tap: the zero piece
-            const bf16x8 B = *(const bf16x8*)(sm + (off[i] >= 0 ? vox[t] + off[i] : HV * SV));
+            const bf16x8 B = *(const bf16x8*)(sm + (off[kc] >= 0 ? vox[t] + off[kc] : HV * SV));
 #pragma unroll
             for (int n = 0; n < NTW; ++n)
                 acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[n], B, acc[t][n], 0, 0, 0);
         }
-    }
-    if constexpr (KS > 1) {
-        f32x4* red = (f32x4*)sm;
-        __syncthreads();
-        if (ks > 0) {
-#pragma unroll
-            for (int t = 0; t < MTW; ++t)
-#pragma unroll
-                for (int n = 0; n < NTW; ++n)
-                    red[(((ks - 1) * WM * WN + wn * WM + wm) * MTW * NTW + t * NTW + n) * 64 + lane] = acc[t][n];
-        }
-        __syncthreads();
-        if (ks > 0) return;
-#pragma unroll
-        for (int j = 0; j < KS - 1; ++j)
-#pragma unroll
-            for (int t = 0; t < MTW; ++t)
-#pragma unroll
-                for (int n = 0; n < NTW; ++n)
-                    acc[t][n] += red[((j * WM * WN + wn * WM + wm) * MTW * NTW + t * NTW + n) * 64 + lane];
     }
     // the lane holds channels 16n + 4g .. + 3 of voxel 16t + m
 #pragma unroll
@@ -647,9 +626,9 @@ template <bool P2>
 __global__ void __launch_bounds__(256) up_kernel(float* __restrict__ p, const float* __restrict__ out,
                                                  const double* __restrict__ stats, float len2, int Zc,
                                                  int Xc, int Yc, int F) {
-    __shared__ double scale;
+    __shared__ double rms;
     if (threadIdx.x == 0 && threadIdx.y == 0)
-        scale = sqrt(stats[1] / ((double)Zc * Xc * Yc)) * (double)len2;
+        rms = sqrt(stats[1] / ((double)Zc * Xc * Yc));
     const int X = Xc * F, Y = Yc * F, Z = Zc * F;
     const int y = blockIdx.x * 64 + threadIdx.x, x = blockIdx.y * 4 + threadIdx.y;
     const float inv_f = 1.f / (float)F;
@@ -679,12 +658,12 @@ __global__ void __launch_bounds__(256) up_kernel(float* __restrict__ p, const fl
         v[k] = (1.f - wz) * v0 + wz * v1;
     }
     __syncthreads();
-    const double sc = scale;
+    const double r = rms;
     if (y >= Y || x >= X) return;
 #pragma unroll
     for (int k = 0; k < kUpZ; ++k) {
         const int64_t z = (int64_t)blockIdx.z * kUpZ + k;
-        if (z < Z) p[y + (int64_t)Y * (x + (int64_t)X * z)] = (float)((double)v[k] * sc);
+        if (z < Z) p[y + (int64_t)Y * (x + (int64_t)X * z)] = (float)((double)v[k] * r * (double)len2);
     }
 }
 
@@ -765,11 +744,11 @@ int check_launch(const char* what) {
 
 dim3 g1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
-template <int CA, int CB, bool UP, int CO, int MODE, int BZ, int BX, int BY, int WM, int WN, int KS>
+template <int CA, int CB, bool UP, int CO, int MODE, int BZ, int BX, int BY, int WM, int WN>
 void conv_launch(const ConvSrc& s, const bf16* w, const ConvOut& o, hipStream_t st) {
     const int64_t bricks = (int64_t)((s.Z + BZ - 1) / BZ) * ((s.X + BX - 1) / BX) * ((s.Y + BY - 1) / BY);
-    hipLaunchKernelGGL((conv3_kernel<CA, CB, UP, CO, MODE, BZ, BX, BY, WM, WN, KS>), dim3((unsigned)bricks),
-                       dim3(64 * WM * WN * KS), 0, st, s, w, o);
+    hipLaunchKernelGGL((conv3_kernel<CA, CB, UP, CO, MODE, BZ, BX, BY, WM, WN>), dim3((unsigned)bricks),
+                       dim3(64 * WM * WN), 0, st, s, w, o);
 }
 
 // Slices of layer l's weight gradient: workgroups for every CU (a slice has one
@@ -791,20 +770,21 @@ void wgrad_launch(whhd_unet_s* h, int l, const ConvSrc& s, const bf16* gy, hipSt
 }
 
 // forward of layer l (RELU into o1, or F32 for the last).  Bricks of 128 voxels
-// on the finest level, 64 and 32 on the coarser ones, whose grids are small;
-// about a dozen chunks of 32 per wavefront.
+// on the finest level, 64 and 16 or 32 on the coarser ones, whose grids are small
+// (64 -> 64 at 12^3, 2 x 2 x 4 voxels and four wavefronts 5.8 us, 2 x 4 x 4 and eight
+// 7.0, and four 10.9); four to twelve wavefronts a brick.
 int fwd_layer(whhd_unet_s* h, int l, const ConvSrc& s, bf16* out_bf, hipStream_t st) {
     ConvOut o{out_bf, nullptr, h->out, h->w + h->boff[l], nullptr, 0};
     const bf16* w = h->wk[l];
     switch (l) {
-    case 0: case 1: case 9: conv_launch<16, 0, false, 16, MODE_RELU, 4, 4, 8, 4, 1, 1>(s, w, o, st); break;
-    case 2: conv_launch<16, 0, false, 32, MODE_RELU, 4, 4, 4, 2, 2, 2>(s, w, o, st); break;
-    case 3: case 7: conv_launch<32, 0, false, 32, MODE_RELU, 4, 4, 4, 2, 2, 2>(s, w, o, st); break;
-    case 4: conv_launch<32, 0, false, 64, MODE_RELU, 2, 4, 4, 1, 4, 3>(s, w, o, st); break;
-    case 5: conv_launch<64, 0, false, 64, MODE_RELU, 2, 4, 4, 1, 4, 4>(s, w, o, st); break;
-    case 6: conv_launch<64, 32, true, 32, MODE_RELU, 4, 4, 4, 1, 2, 6>(s, w, o, st); break;
-    case 8: conv_launch<32, 16, true, 16, MODE_RELU, 4, 4, 8, 2, 1, 4>(s, w, o, st); break;
-    default: conv_launch<16, 0, false, 16, MODE_F32, 4, 4, 8, 4, 1, 1>(s, w, o, st); break;
+    case 0: case 1: case 9: conv_launch<16, 0, false, 16, MODE_RELU, 4, 4, 8, 4, 1>(s, w, o, st); break;
+    case 2: conv_launch<16, 0, false, 32, MODE_RELU, 4, 4, 4, 4, 2>(s, w, o, st); break;
+    case 3: case 7: conv_launch<32, 0, false, 32, MODE_RELU, 4, 4, 4, 4, 2>(s, w, o, st); break;
+    case 4: conv_launch<32, 0, false, 64, MODE_RELU, 2, 2, 4, 1, 4>(s, w, o, st); break;
+    case 5: conv_launch<64, 0, false, 64, MODE_RELU, 2, 2, 4, 1, 4>(s, w, o, st); break;
+    case 6: conv_launch<64, 32, true, 32, MODE_RELU, 4, 4, 4, 4, 2>(s, w, o, st); break;
+    case 8: conv_launch<32, 16, true, 16, MODE_RELU, 4, 4, 8, 4, 1>(s, w, o, st); break;
+    default: conv_launch<16, 0, false, 16, MODE_F32, 4, 4, 8, 4, 1>(s, w, o, st); break;
     }
     return check_launch("unet_conv3_kernel");
 }
@@ -818,13 +798,13 @@ int bwd_data(whhd_unet_s* h, int l, const bf16* G, int Z, int X, int Y, bf16* o1
     const ConvOut o{o1, o2, nullptr, nullptr, mask, split};
     const bf16* w = h->wt[l];
     switch (l) {
-    case 1: case 9: case 10: conv_launch<16, 0, false, 16, MODE_GRAD, 4, 4, 8, 4, 1, 1>(s, w, o, st); break;
-    case 2: conv_launch<32, 0, false, 16, MODE_GRAD, 4, 4, 4, 4, 1, 2>(s, w, o, st); break;
-    case 3: case 7: conv_launch<32, 0, false, 32, MODE_GRAD, 4, 4, 4, 2, 2, 2>(s, w, o, st); break;
-    case 4: conv_launch<64, 0, false, 32, MODE_GRAD, 2, 4, 4, 1, 2, 6>(s, w, o, st); break;
-    case 5: conv_launch<64, 0, false, 64, MODE_GRAD, 2, 4, 4, 1, 4, 4>(s, w, o, st); break;
-    case 6: conv_launch<32, 0, false, 96, MODE_GRAD, 4, 4, 4, 1, 6, 2>(s, w, o, st); break;
-    case 8: conv_launch<16, 0, false, 48, MODE_GRAD, 4, 4, 8, 4, 1, 1>(s, w, o, st); break;
+    case 1: case 9: case 10: conv_launch<16, 0, false, 16, MODE_GRAD, 4, 4, 8, 4, 1>(s, w, o, st); break;
+    case 2: conv_launch<32, 0, false, 16, MODE_GRAD, 4, 4, 4, 4, 1>(s, w, o, st); break;
+    case 3: case 7: conv_launch<32, 0, false, 32, MODE_GRAD, 4, 4, 4, 4, 2>(s, w, o, st); break;
+    case 4: conv_launch<64, 0, false, 32, MODE_GRAD, 2, 4, 4, 2, 2>(s, w, o, st); break;
+    case 5: conv_launch<64, 0, false, 64, MODE_GRAD, 2, 2, 4, 1, 4>(s, w, o, st); break;
+    case 6: conv_launch<32, 0, false, 96, MODE_GRAD, 4, 4, 4, 2, 6>(s, w, o, st); break;
+    case 8: conv_launch<16, 0, false, 48, MODE_GRAD, 4, 4, 8, 4, 1>(s, w, o, st); break;
     default: return fail(WHHD_INVALID_ARG, "unet: no input gradient for the first layer");
     }
     return check_launch("unet_conv3_kernel(grad)");
